@@ -22,6 +22,7 @@ NXA_F16 = 2
 NXA_WS_FWD = 0
 NXA_WS_BWD = 1
 NXA_WS_DBIAS = 2
+NXA_WS_PACK = 8
 
 # static scratch of nxa_fwd_noalloc (NXA_NOALLOC_SCRATCH_BYTES)
 NXA_NOALLOC_SCRATCH_BYTES = 8 << 20

@@ -431,7 +431,9 @@ def _forward(prep: _Prepared, for_bwd: bool = False, qnorm=None):
     lse = torch.empty(
         (prep.nb, prep.h, prep.s), dtype=torch.float32, device=prep.device
     )
-    ws = prep.workspace(_lib.NXA_WS_BWD if for_bwd else _lib.NXA_WS_FWD)
+    # Room for the packed bias (nxa_fwd_normed has no use for it).
+    pack = _lib.NXA_WS_PACK if qnorm is None else 0
+    ws = prep.workspace((_lib.NXA_WS_BWD if for_bwd else _lib.NXA_WS_FWD) | pack)
     args = (ctypes.byref(prep.desc), _ptr(prep.q), _ptr(prep.k), _ptr(prep.v),
             _ptr(prep.bias), _ptr(prep.mask), _ptr(o), _ptr(lse))
     tail = (_ptr(ws), 0 if ws is None else ws.numel(), prep.stream())
@@ -488,6 +490,8 @@ def _backward(prep: _Prepared, o, lse, fwd_ws, dout, want_dbias: bool, norm=None
     # The workspace begins with the forward's tile map; a forward workspace
     # already sized for this backward is reused in place.
     flags = _lib.NXA_WS_BWD | (_lib.NXA_WS_DBIAS if dbias is not None else 0)
+    if norm is None:
+        flags |= _lib.NXA_WS_PACK
     need = prep.workspace_bytes(flags)
     ready = 0
     if fwd_ws is not None and fwd_ws.numel() >= need:

@@ -228,14 +228,48 @@ DbiasGeom dbias_geom(const nxa_desc* d) {
   return g;
 }
 
+// Short-sequence path (nxa_short16.hip): 16-bit I/O, both head dims at most
+// 64, at most kShortMax queries and keys, a mask (if any) that broadcasts
+// over queries, and a bias (if any) shared by at least four (batch, head)
+// pairs, so that packing it costs less than the pairs' reads of it, with a
+// positive scale whose reciprocal is far from the ends of fp32's range.
+// Decided on the descriptor alone, so that a call's forward, backward and
+// workspace sizes agree.
+struct ShortGeom {
+  bool ok;
+  int OB, OH, nqb, nkb;
+  size_t pack_bytes;  // one layout of the packed bias
+};
+
+ShortGeom short_geom(const nxa_desc* d, int has_bias, int has_mask) {
+  ShortGeom g{};
+  const int64_t kRow = 1 << 21;  // resident rows are addressed with 32-bit offsets
+  g.ok = d->io_dtype != NXA_F32 && d->D <= 64 && value_dim(d) <= 64 &&
+         d->Lq <= nxa::kShortMax && d->Lk <= nxa::kShortMax && d->q_str[2] <= kRow &&
+         d->k_str[2] <= kRow && d->v_str[2] <= kRow && d->o_str[2] <= kRow && d->scale > 1e-6f &&
+         d->scale < 1e6f;
+  if (has_mask && d->mask_str[2] != 0 && d->Lq > 1) g.ok = false;
+  g.OB = g.OH = 1;
+  g.nqb = 2 * ((d->Lq + 63) / 64);
+  g.nkb = 2 * ((d->Lk + 63) / 64);
+  if (has_bias) {
+    g.OB = d->bias_str[0] == 0 ? 1 : d->B;
+    g.OH = d->bias_str[1] == 0 ? 1 : d->H;
+    if ((int64_t)d->B * d->H < 4 * (int64_t)g.OB * g.OH) g.ok = false;
+    g.pack_bytes = (size_t)g.OB * g.OH * g.nqb * g.nkb * 1024 * sizeof(float);
+  }
+  return g;
+}
+
 struct WsLayout {
-  size_t tilemap, order, delta, acc, partial, total;
+  size_t tilemap, order, pack, delta, acc, partial, total;
 };
 
 // flags: NXA_WS_BWD (bit 0) sizes the backward's per-row values, and
 // NXA_WS_DBIAS (bit 1) its dbias reduction buffers.
+// NXA_WS_PACK adds the packed bias of the short-sequence kernels.
 WsLayout ws_layout(const nxa_desc* d, int has_bias, int has_mask, int flags) {
-  WsLayout w{0, 0, 0, 0, 0, 0};
+  WsLayout w{};
   size_t off = 0;
   if (has_mask) {
     const MaskGeom m = mask_geom(d);
@@ -243,6 +277,12 @@ WsLayout ws_layout(const nxa_desc* d, int has_bias, int has_mask, int flags) {
     off += align256(m.bytes);
     w.order = off;
     off += align256(m.order_bytes);
+  }
+  if (has_bias && (flags & NXA_WS_PACK)) {
+    // Packed bias: the S^T layout, and in the backward the S layout after it.
+    const ShortGeom g = short_geom(d, has_bias, has_mask);
+    w.pack = off;
+    if (g.ok) off += (flags & NXA_WS_BWD ? 2 : 1) * align256(g.pack_bytes);
   }
   if (flags & NXA_WS_BWD) {
     w.delta = off;  // -delta[B*H*Lq], then -lse2[B*H*Lq]
@@ -359,6 +399,18 @@ nxa::Params base_params(const nxa_desc* d, const void* q, const void* k,
     p.mask_vec = vec;
   }
   return p;
+}
+
+nxa::ShortParams short_params(const nxa_desc* d, const ShortGeom& g, uint8_t* pack, bool bwd) {
+  nxa::ShortParams sp{};
+  sp.OB = g.OB;
+  sp.OH = g.OH;
+  sp.nqb = g.nqb;
+  sp.nkb = g.nkb;
+  sp.inv_scale = 1.0f / d->scale;
+  sp.pack_st = reinterpret_cast<float*>(pack);
+  if (bwd) sp.pack_s = reinterpret_cast<float*>(pack + align256(g.pack_bytes));
+  return sp;
 }
 
 // Writes (or just binds) the tile map for `mask`, and the block order when
@@ -511,9 +563,10 @@ struct FwdNorm {
   float eps;
 };
 
+// `packs`: the workspace has room for the packed bias.
 int run_fwd(const nxa_desc* d, const void* q, const void* k, const void* v,
             const void* bias, const uint8_t* mask, void* o, float* lse,
-            void* workspace, void* stream_, const FwdNorm* fn = nullptr);
+            void* workspace, bool packs, void* stream_, const FwdNorm* fn = nullptr);
 
 // ---------------------------------------------------------------------------
 // Static scratch of nxa_fwd_noalloc: a device array that every GPU the
@@ -565,8 +618,8 @@ int nxa_check(const nxa_desc* desc, int has_bias, int has_mask) {
 size_t nxa_workspace_bytes(const nxa_desc* desc, int has_bias, int has_mask,
                            int flags) {
   if (check_desc(desc, has_bias, has_mask) != NXA_OK) return 0;
-  if (flags & ~(NXA_WS_BWD | NXA_WS_DBIAS)) {
-    fail(NXA_E_ARG, "workspace flags %d: only NXA_WS_BWD | NXA_WS_DBIAS", flags);
+  if (flags & ~(NXA_WS_BWD | NXA_WS_DBIAS | NXA_WS_PACK)) {
+    fail(NXA_E_ARG, "workspace flags %d: only NXA_WS_BWD | NXA_WS_DBIAS | NXA_WS_PACK", flags);
     return 0;
   }
   return ws_layout(desc, has_bias, has_mask, flags).total;
@@ -577,11 +630,14 @@ int nxa_fwd(const nxa_desc* d, const void* q, const void* k, const void* v,
             void* workspace, size_t workspace_bytes, void* stream_) {
   int rc = check_fwd(d, q, k, v, bias, mask, o);
   if (rc) return rc;
+  // Without room for the packed bias the general kernels take the call.
   const WsLayout ws = ws_layout(d, bias != nullptr, mask != nullptr, 0);
   if (ws.total > 0 && (!workspace || workspace_bytes < ws.total))
     return fail(NXA_E_WORKSPACE, "forward needs %zu workspace bytes, got %zu",
                 ws.total, workspace ? workspace_bytes : (size_t)0);
-  return run_fwd(d, q, k, v, bias, mask, o, lse, workspace, stream_);
+  const size_t full = ws_layout(d, bias != nullptr, mask != nullptr, NXA_WS_PACK).total;
+  return run_fwd(d, q, k, v, bias, mask, o, lse, workspace,
+                 workspace && workspace_bytes >= full, stream_);
 }
 
 int nxa_fwd_normed(const nxa_desc* d, const void* q, const void* k_hat, const void* v,
@@ -604,7 +660,7 @@ int nxa_fwd_normed(const nxa_desc* d, const void* q, const void* k_hat, const vo
     return fail(NXA_E_WORKSPACE, "forward needs %zu workspace bytes, got %zu",
                 ws.total, workspace ? workspace_bytes : (size_t)0);
   const FwdNorm fn{q_hat, q_rstd, eps};
-  return run_fwd(d, q, k_hat, v, bias, mask, o, lse, workspace, stream_, &fn);
+  return run_fwd(d, q, k_hat, v, bias, mask, o, lse, workspace, false, stream_, &fn);
 }
 
 int nxa_fwd_noalloc(const nxa_desc* d, const void* q, const void* k, const void* v,
@@ -620,18 +676,19 @@ int nxa_fwd_noalloc(const nxa_desc* d, const void* q, const void* k, const void*
                 ws.total, kScratchBytes);
   void* scratch_ptr = nullptr;
   if (ws.total > 0 && (rc = device_scratch(&scratch_ptr))) return rc;
-  return run_fwd(d, q, k, v, bias, mask, o, lse, scratch_ptr, stream_);
+  return run_fwd(d, q, k, v, bias, mask, o, lse, scratch_ptr, false, stream_);
 }
 
 }  // extern "C"
 
 namespace {
 
-// The forward after validation: tile map into `workspace` (when there is a
-// mask), then the forward kernel.
+// The forward after validation: the short-sequence kernels where they take
+// the problem (after packing a bias into `workspace`), else the tile map into
+// `workspace` (when there is a mask) and the forward kernel.
 int run_fwd(const nxa_desc* d, const void* q, const void* k, const void* v,
             const void* bias, const uint8_t* mask, void* o, float* lse,
-            void* workspace, void* stream_, const FwdNorm* fn) {
+            void* workspace, bool packs, void* stream_, const FwdNorm* fn) {
   int rc;
   hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
   nxa::Params p = base_params(d, q, k, v, bias, mask);
@@ -642,6 +699,22 @@ int run_fwd(const nxa_desc* d, const void* q, const void* k, const void* v,
     p.qn_out = fn->q_hat;
     p.qn_rstd = fn->q_rstd;
     p.qn_eps = fn->eps;
+  }
+  const ShortGeom sg = short_geom(d, bias != nullptr, mask != nullptr);
+  // A bias that the general forward adds on the matrix cores straight from
+  // its rows saves the pack, which up to 256 pairs costs more than the
+  // short kernels gain (head dim 64, 64 pairs of 512 x 512: 18.3 us general,
+  // 22.7 packed; 256 pairs: 38 and 44; 512 pairs of 400 x 400: 74 and 67).
+  const bool direct = bias && p.fwd_bias != nxa::kFbValu && (int64_t)d->B * d->H <= 256;
+  if (sg.ok && !fn && !direct && (!bias || packs)) {
+    const WsLayout w = ws_layout(d, bias != nullptr, mask != nullptr, NXA_WS_PACK);
+    const nxa::ShortParams sp =
+        short_params(d, sg, bias ? static_cast<uint8_t*>(workspace) + w.pack : nullptr, false);
+    if (bias &&
+        (rc = launch("bias_pack", stream, [&] { nxa::launch_bias_pack(p, sp, stream); })))
+      return rc;
+    return launch("fwd", stream,
+                  [&] { nxa::launch_short(p, sp, d->io_dtype, nxa::kShortFwd, stream); });
   }
   if (mask) {
     rc = setup_tilemap(p, d, static_cast<uint8_t*>(workspace), true, stream);
@@ -691,8 +764,15 @@ int run_bwd(const nxa_desc* d, const void* q, const void* k, const void* v,
       return fail(NXA_E_UNSUPPORTED,
                   "backward needs q materialised over axis %d (stride 0)", i);
   }
-  const WsLayout ws = ws_layout(d, bias != nullptr, mask != nullptr,
-                                NXA_WS_BWD | (dbias ? NXA_WS_DBIAS : 0));
+  const int ws_flags = NXA_WS_BWD | (dbias ? NXA_WS_DBIAS : 0);
+  WsLayout ws = ws_layout(d, bias != nullptr, mask != nullptr, ws_flags | NXA_WS_PACK);
+  const ShortGeom sg = short_geom(d, bias != nullptr, mask != nullptr);
+  bool use_short = sg.ok && !na;
+  if (!workspace || workspace_bytes < ws.total || !use_short) {
+    // No room for the packed bias (or no use for it): the general kernels.
+    use_short = use_short && !bias;
+    ws = ws_layout(d, bias != nullptr, mask != nullptr, ws_flags);
+  }
   if (!workspace || workspace_bytes < ws.total)
     return fail(NXA_E_WORKSPACE, "backward needs %zu workspace bytes, got %zu",
                 ws.total, workspace ? workspace_bytes : (size_t)0);
@@ -708,6 +788,52 @@ int run_bwd(const nxa_desc* d, const void* q, const void* k, const void* v,
   p.ndelta = reinterpret_cast<float*>(wsb + ws.delta);
   p.nlse2 = reinterpret_cast<float*>(
       wsb + ws.delta + align256((size_t)d->B * d->H * d->Lq * sizeof(float)));
+  if (use_short) {
+    DbiasGeom dg{};
+    nxa::ShortParams sp = short_params(d, sg, bias ? wsb + ws.pack : nullptr, true);
+    if (dbias) {
+      // The slabs take the place of the accumulator and the partials (one
+      // region, ws.acc onwards): as many ranges as fit there and keep the
+      // grid within the blocks the chip holds at once (three a CU at head
+      // dim 32, one at 64).
+      dg = dbias_geom(d);
+      sp.slabs = reinterpret_cast<float*>(wsb + ws.acc);
+      sp.Lkp = (d->Lk + 3) & ~3;
+      const int64_t slots = (int64_t)sg.OB * sg.OH, pairs = (int64_t)d->B * d->H / slots;
+      const int dp = d->D <= 32 && value_dim(d) <= 32 ? 32 : 64;
+      const int64_t tiles = slots * nxa::short_dbias_tiles(d->Lq, d->Lk, dp);
+      const int64_t room = dp == 32 ? 768 : 256;
+      const int64_t slab = slots * d->Lq * sp.Lkp * (int64_t)sizeof(float);
+      int64_t n = tiles < room ? room / tiles : 1;
+      const int64_t fit = (int64_t)(ws.total - ws.acc) / slab;
+      if (n > fit) n = fit;
+      if (n > pairs) n = pairs;
+      sp.nrange = (int)n;
+    }
+    // A column-sum dbias (a bias that broadcasts over queries) and a region
+    // too small for one slab stay with the general kernels.
+    if (!dbias || (dg.mode == nxa::kDbiasFull && sp.nrange > 0)) {
+      if (bias &&
+          (rc = launch("bias_pack", stream, [&] { nxa::launch_bias_pack(p, sp, stream); })))
+        return rc;
+      const struct {
+        const char* name;
+        nxa::ShortPart part;
+      } parts[3] = {{"dq", nxa::kShortDq}, {"dkdv", nxa::kShortDkdv}, {"dbias", nxa::kShortDbias}};
+      for (int i = 0; i < (dbias ? 3 : 2); ++i)
+        if ((rc = launch(parts[i].name, stream, [&] {
+               nxa::launch_short(p, sp, d->io_dtype, parts[i].part, stream);
+             })))
+          return rc;
+      if (dbias)
+        return launch("dbias_reduce", stream, [&] {
+          nxa::launch_dbias_slabs(p, sp, dbias, dbias_str, stream);
+        });
+      return NXA_OK;
+    }
+  }
+  // A forward on the short-sequence kernels leaves no tile map behind.
+  if (sg.ok) tilemap_ready = 0;
   // 16-bit I/O: the dQ kernel computes -delta and -lse * log2(e) for its own
   // rows and runs first; the fp32 kernels have a pass of its own.
   const bool dq_first = d->io_dtype != NXA_F32;

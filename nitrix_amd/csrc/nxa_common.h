@@ -380,6 +380,12 @@ template <>
 __device__ __forceinline__ int swz<64>(int r) {
   return 4 * ((r >> 1) & 1) + ((r >> 2) & 3);
 }
+// 32 columns: 16 rows of one chunk fill four 256-byte bank rows, each with
+// the chunk at four different places; 4 rows x 64 bytes are one bank row.
+template <>
+__device__ __forceinline__ int swz<32>(int r) {
+  return (r >> 2) & 3;
+}
 template <int DP>
 __device__ __forceinline__ int swz_off(int row, int chunk) {
   return row * DP + 8 * (chunk ^ swz<DP>(row));

@@ -28,6 +28,30 @@ void launch_dq16(const Params& p, int io_dtype, int dp, hipStream_t stream);
 void launch_fwd16_wide(const Params& p, int io_dtype, hipStream_t stream);
 void launch_dkdv16_wide(const Params& p, int io_dtype, hipStream_t stream);
 void launch_dq16_wide(const Params& p, int io_dtype, hipStream_t stream);
+// Short-sequence kernels (nxa_short16.hip).
+constexpr int kShortMax = 512;  // queries and keys
+struct ShortParams {
+  int OB, OH;        // extents of the bias over batch / heads (1: broadcast)
+  int nqb, nkb;      // packed 32-query / 32-key blocks (an even count each)
+  float inv_scale;
+  float* pack_st;    // [OB][OH][nqb][nkb][1024] bias / scale, S^T accumulator layout
+  float* pack_s;     // the same, S layout (backward; may be null in the forward)
+  float* slabs;      // [nrange][OB][OH][Lq][Lkp] fp32 sums of dS (dbias)
+  int nrange, Lkp;
+  int nsplit;        // blocks per (batch, head) pair (set by the launcher)
+};
+// Blocks of the dbias kernel over one bias slot (128 queries x 64 keys at
+// padded head dim 32, 128 x 128 at 64).
+inline int short_dbias_tiles(int Lq, int Lk, int dp) {
+  const int bk = dp == 32 ? 64 : 128;
+  return ((Lq + 127) / 128) * ((Lk + bk - 1) / bk);
+}
+enum ShortPart : int { kShortFwd, kShortDq, kShortDkdv, kShortDbias };
+void launch_short(const Params& p, const ShortParams& sp, int io_dtype, ShortPart part,
+                  hipStream_t stream);
+void launch_bias_pack(const Params& p, const ShortParams& sp, hipStream_t stream);
+void launch_dbias_slabs(const Params& p, const ShortParams& sp, void* out, const int64_t* str,
+                        hipStream_t stream);
 void launch_rms_norm(const NormParams& p, int dtype, bool bwd, hipStream_t stream);
 int ssm_padded_states(int N);
 int ssm_lanes_per_channel(int NP);

@@ -1,0 +1,94 @@
+"""Parity of the short-sequence kernels (at most 512 queries and keys, head
+dims up to 64, 16-bit I/O) against the float64 oracle, at the edges of their
+strips, tiles and limits: lengths around 32 and 64 rows and at 512, head dims
+around the 32-wide variant, a bias shared by many pairs in every broadcast
+pattern and dtype (odd row lengths, so that nothing is aligned), key padding
+over an odd length, causal with s != t, and the first lengths and shapes the
+general kernels take again."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+from test_hip_parity import _check, _dev, _draw, _to
+
+pytestmark = pytest.mark.gpu
+
+BF, HF, F32 = torch.bfloat16, torch.float16, torch.float32
+
+
+@pytest.mark.parametrize('dtype', [BF, HF], ids=['bf16', 'f16'])
+@pytest.mark.parametrize('s, t, d, dv', [
+    (5, 7, 8, 8), (31, 33, 32, 32), (64, 65, 40, 40), (95, 129, 32, 64), (343, 343, 32, 32),
+    (512, 512, 64, 64), (512, 513, 64, 64), (513, 300, 24, 24), (300, 17, 64, 16),
+])
+def test_lengths_and_head_dims(dtype, s, t, d, dv):
+    _check(dtype, 3, 4, s, t, d, dv=dv, seed=s + t + d)
+    _check(dtype, 3, 4, s, t, d, dv=dv, mask_kind='keypad', seed=s + t)
+    _check(dtype, 2, 4, s, t, d, dv=dv, causal=True, seed=s)
+
+
+@pytest.mark.parametrize('bias_dtype', [BF, F32], ids=['bf16', 'f32'])
+@pytest.mark.parametrize('B, H, bias', [
+    (8, 3, (3, 0, 0)), (4, 5, (1, 1, 0, 0)), (3, 8, (3, 1, 0, 0)), (5, 2, (1, 2, 1, 0)),
+    (64, 4, (4, 0, 0)), (3, 3, (3, 0, 0)),
+], ids=['heads', 'one', 'batch', 'row', 'many', 'share3'])
+@pytest.mark.parametrize('s, t, d', [(49, 49, 32), (343, 343, 32), (100, 130, 64), (33, 511, 48)])
+def test_shared_bias(bias_dtype, B, H, bias, s, t, d):
+    shape = tuple(n or m for n, m in zip(bias, (*(1,) * (len(bias) - 2), s, t)))
+    _check(BF, B, H, s, t, d, bias_shape=shape, bias_dtype=bias_dtype, seed=s + B)
+    if B < 64:
+        _check(BF, B, H, s, t, d, bias_shape=shape, bias_dtype=bias_dtype, mask_kind='keypad',
+               causal=s == t, scale=0.3, seed=t + B)
+
+
+@pytest.mark.parametrize('dtype', [BF, HF], ids=['bf16', 'f16'])
+def test_large_and_negative_infinite_bias(dtype):
+    """A shared bias used as a mask (-inf on some keys of every row) and one
+    whose logits rise far above the first tiles' (the row reference moves)."""
+    rng = np.random.default_rng(3)
+    B, H, s, t, d = 4, 2, 100, 201, 32
+    q, k, v = (_draw(rng, (B, H, n, d), dtype) for n in (s, t, t))
+    bias = np.linspace(0, 300, t, dtype=np.float32)[None, None] + np.zeros((H, s, 1), np.float32)
+    bias = bias.astype(np.float16).astype(np.float32) if dtype == HF else np.floor(bias)
+    bias[:, :, 1::3] = -np.inf
+    from nitrix_amd import scaled_dot_product_attention
+    from oracle import attention as O
+
+    if dtype == BF:
+        bias = O.round_bf16(np.where(np.isinf(bias), 0, bias)).astype(np.float32)
+        bias[:, :, 1::3] = -np.inf
+    out = scaled_dot_product_attention(_to(q, dtype), _to(k, dtype), _to(v, dtype),
+                                       bias=_to(bias, dtype), backend='hip')
+    ref = O.sdpa_forward(q, k, v, bias=bias, scale=d ** -0.5, acc_dtype=np.float64)
+    got = out.float().cpu().numpy()
+    assert np.isfinite(got).all()
+    assert np.abs(got - ref).max() / np.abs(ref).max() <= (2e-2 if dtype == BF else 2e-3)
+
+
+def test_workspace_without_room_for_the_packed_bias():
+    """A caller that passes no workspace to a mask-free forward with a shared
+    bias is served by the general kernels, to rounding."""
+    import ctypes
+
+    from nitrix_amd import _lib
+    from nitrix_amd.attention import _Prepared
+
+    g = torch.Generator(device=_dev()).manual_seed(5)
+    q, k, v = (torch.randn(8, 2, 70, 32, generator=g, device=_dev()).to(BF) for _ in range(3))
+    bias = torch.randn(2, 70, 70, generator=g, device=_dev()).to(BF)
+    prep = _Prepared(q, k, v, bias, None, 32 ** -0.5, False)
+    outs = []
+    for ws in (prep.workspace(_lib.NXA_WS_PACK), None):
+        o = torch.empty_like(q)
+        lse = torch.empty(8, 2, 70, device=_dev())
+        _lib.check(_lib.lib().nxa_fwd(
+            ctypes.byref(prep.desc), prep.q.data_ptr(), prep.k.data_ptr(), prep.v.data_ptr(),
+            prep.bias.data_ptr(), None, o.data_ptr(), lse.data_ptr(),
+            None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
+            prep.stream()))
+        outs.append((o.float(), lse))
+    assert prep.workspace_bytes(_lib.NXA_WS_PACK) > prep.workspace_bytes(_lib.NXA_WS_FWD) == 0
+    torch.testing.assert_close(outs[0][0], outs[1][0], rtol=0, atol=2e-2)
+    torch.testing.assert_close(outs[0][1], outs[1][1], rtol=0, atol=2e-3)
