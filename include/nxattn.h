@@ -55,7 +55,7 @@ extern "C" {
 #define NXA_WS_FWD 0   /* the forward                                        */
 #define NXA_WS_BWD 1   /* the backward                                       */
 #define NXA_WS_DBIAS 2 /* with NXA_WS_BWD: a backward that writes dbias      */
-#define NXA_WS_PACK 8  /* room for the packed bias of short sequences (below) */
+#define NXA_WS_PACK 8  /* room for a packed bias or key splits (below)         */
 
 typedef enum { NXA_BF16 = 0, NXA_F32 = 1, NXA_F16 = 2 } nxa_dtype;
 
@@ -111,8 +111,11 @@ int nxa_check(const nxa_desc* desc, int has_bias, int has_mask);
  * and keys and head dims of at most 64 whose bias is shared by at least four
  * (batch, head) pairs (and whose mask, if any, broadcasts over queries),
  * room for the bias packed in fp32 (padded to whole 64 x 64 tiles; twice in
- * the backward); without that room such a problem is taken by the general
- * kernels, which read the bias as it is.  A workspace sized for the backward also serves the forward.
+ * the backward), and for a forward of at most 64 queries over more than 512
+ * keys (bf16 / fp16, head dims of at most 128, no bias, not causal, the same
+ * masks) room for the partial results of its key splits (fp32, one padded
+ * output per 32 queries and split); without that room such a problem is
+ * taken by the general kernels.  A workspace sized for the backward also serves the forward.
  * Returns 0 for an invalid descriptor or flags. */
 size_t nxa_workspace_bytes(const nxa_desc* desc, int has_bias, int has_mask,
                            int flags);
@@ -121,8 +124,8 @@ size_t nxa_workspace_bytes(const nxa_desc* desc, int has_bias, int has_mask,
  * bias / mask may be NULL; lse may be NULL.  When mask is given, the first
  * nxa_workspace_bytes(desc, .., 0) bytes of the workspace receive the
  * tile map (and block order) that nxa_bwd can reuse (tilemap_ready = 1);
- * problems of at most 512 queries and keys may leave it unwritten, and
- * nxa_bwd then does not read it either. */
+ * problems of at most 512 queries and keys, or of at most 64 queries, may
+ * leave it unwritten, and nxa_bwd then does not read it either. */
 int nxa_fwd(const nxa_desc* desc, const void* q, const void* k, const void* v,
             const void* bias, const uint8_t* mask, void* o, float* lse,
             void* workspace, size_t workspace_bytes, void* stream);
@@ -131,8 +134,8 @@ int nxa_fwd(const nxa_desc* desc, const void* q, const void* k, const void* v,
  * the reference: it is for callers that cannot allocate device memory at all
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  The same kernels and results as nxa_fwd (where that would
- * pack a shared bias into its workspace, the general kernels instead, which
- * agree to rounding); the mask's tile map
+ * use the room of NXA_WS_PACK, the general kernels instead, which agree to
+ * rounding); the mask's tile map
  * (and block order) goes to a static device array of NXA_NOALLOC_SCRATCH_BYTES
  * that every GPU the library runs on holds until the process ends.  A tile
  * map larger than that (nxa_workspace_bytes(desc, .., NXA_WS_FWD)) is

@@ -261,13 +261,45 @@ ShortGeom short_geom(const nxa_desc* d, int has_bias, int has_mask) {
   return g;
 }
 
+// Key-split forward (nxa_split16.hip): 16-bit I/O, at most kSplitMaxQ queries
+// over more keys than the short-sequence kernels take, no bias, not causal,
+// a mask (if any) that broadcasts over queries.  On the descriptor alone, as
+// short_geom.
+struct SplitGeom {
+  bool ok;
+  int dp, strips, splits;
+  size_t part_bytes;
+};
+
+SplitGeom split_geom(const nxa_desc* d, int has_bias, int has_mask) {
+  SplitGeom g{};
+  const int m = d->D > value_dim(d) ? d->D : value_dim(d);
+  const int64_t kRow = 1 << 21;
+  g.ok = d->io_dtype != NXA_F32 && !has_bias && !d->causal && m <= 128 &&
+         d->Lq <= nxa::kSplitMaxQ && d->Lk >= nxa::kSplitMinK && d->k_str[2] <= kRow &&
+         d->v_str[2] <= kRow && !(has_mask && d->mask_str[2] != 0 && d->Lq > 1);
+  if (!g.ok) return g;
+  g.dp = m <= 32 ? 32 : m <= 64 ? 64 : 128;
+  g.strips = (d->Lq + 31) / 32;
+  const int64_t strips = (int64_t)d->B * d->H * g.strips;
+  // A second strip reads the keys again: worth it only while the pairs alone
+  // leave CUs idle (B 16, H 32, 64 queries, 1024 keys, head dim 128: 61 us on
+  // the general kernel, 90 split; B 8, H 16, 2048 keys, 64: 37 and 30).
+  if (g.strips > 1 && (int64_t)d->B * d->H > 128) g.ok = false;
+  g.splits = nxa::split_count(strips, d->Lk);
+  if (strips * g.splits * 16 >= (int64_t)1 << 31) g.ok = false;  // the grids
+  if (g.splits > 1) g.part_bytes = (size_t)(strips * g.splits) * nxa::split_part_bytes(g.dp);
+  return g;
+}
+
 struct WsLayout {
   size_t tilemap, order, pack, delta, acc, partial, total;
 };
 
 // flags: NXA_WS_BWD (bit 0) sizes the backward's per-row values, and
 // NXA_WS_DBIAS (bit 1) its dbias reduction buffers.
-// NXA_WS_PACK adds the packed bias of the short-sequence kernels.
+// NXA_WS_PACK adds the packed bias of the short-sequence kernels or the
+// partial results of the key-split forward.
 WsLayout ws_layout(const nxa_desc* d, int has_bias, int has_mask, int flags) {
   WsLayout w{};
   size_t off = 0;
@@ -283,6 +315,11 @@ WsLayout ws_layout(const nxa_desc* d, int has_bias, int has_mask, int flags) {
     const ShortGeom g = short_geom(d, has_bias, has_mask);
     w.pack = off;
     if (g.ok) off += (flags & NXA_WS_BWD ? 2 : 1) * align256(g.pack_bytes);
+  }
+  if (!has_bias && (flags & NXA_WS_PACK)) {
+    // Partial results of the key-split forward (never beside a packed bias).
+    w.pack = off;
+    off += align256(split_geom(d, has_bias, has_mask).part_bytes);
   }
   if (flags & NXA_WS_BWD) {
     w.delta = off;  // -delta[B*H*Lq], then -lse2[B*H*Lq]
@@ -563,7 +600,7 @@ struct FwdNorm {
   float eps;
 };
 
-// `packs`: the workspace has room for the packed bias.
+// `packs`: the workspace has the room of NXA_WS_PACK.
 int run_fwd(const nxa_desc* d, const void* q, const void* k, const void* v,
             const void* bias, const uint8_t* mask, void* o, float* lse,
             void* workspace, bool packs, void* stream_, const FwdNorm* fn = nullptr);
@@ -630,14 +667,15 @@ int nxa_fwd(const nxa_desc* d, const void* q, const void* k, const void* v,
             void* workspace, size_t workspace_bytes, void* stream_) {
   int rc = check_fwd(d, q, k, v, bias, mask, o);
   if (rc) return rc;
-  // Without room for the packed bias the general kernels take the call.
+  // Without room for the packed bias or the partial results of key splits the
+  // general kernels take the call.
   const WsLayout ws = ws_layout(d, bias != nullptr, mask != nullptr, 0);
   if (ws.total > 0 && (!workspace || workspace_bytes < ws.total))
     return fail(NXA_E_WORKSPACE, "forward needs %zu workspace bytes, got %zu",
                 ws.total, workspace ? workspace_bytes : (size_t)0);
   const size_t full = ws_layout(d, bias != nullptr, mask != nullptr, NXA_WS_PACK).total;
   return run_fwd(d, q, k, v, bias, mask, o, lse, workspace,
-                 workspace && workspace_bytes >= full, stream_);
+                 full == 0 || (workspace && workspace_bytes >= full), stream_);
 }
 
 int nxa_fwd_normed(const nxa_desc* d, const void* q, const void* k_hat, const void* v,
@@ -715,6 +753,15 @@ int run_fwd(const nxa_desc* d, const void* q, const void* k, const void* v,
       return rc;
     return launch("fwd", stream,
                   [&] { nxa::launch_short(p, sp, d->io_dtype, nxa::kShortFwd, stream); });
+  }
+  const SplitGeom kg = split_geom(d, bias != nullptr, mask != nullptr);
+  if (kg.ok && !fn && (packs || kg.splits == 1)) {
+    const WsLayout w = ws_layout(d, bias != nullptr, mask != nullptr, NXA_WS_PACK);
+    const nxa::SplitParams kp{
+        kg.strips, kg.splits,
+        kg.splits > 1 ? reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + w.pack) : nullptr};
+    return launch("fwd", stream,
+                  [&] { nxa::launch_fwd_split(p, kp, d->io_dtype, kg.dp, stream); });
   }
   if (mask) {
     rc = setup_tilemap(p, d, static_cast<uint8_t*>(workspace), true, stream);
@@ -832,8 +879,8 @@ int run_bwd(const nxa_desc* d, const void* q, const void* k, const void* v,
       return NXA_OK;
     }
   }
-  // A forward on the short-sequence kernels leaves no tile map behind.
-  if (sg.ok) tilemap_ready = 0;
+  // A forward on the short-sequence or key-split kernels leaves no tile map.
+  if (sg.ok || split_geom(d, bias != nullptr, mask != nullptr).ok) tilemap_ready = 0;
   // 16-bit I/O: the dQ kernel computes -delta and -lse * log2(e) for its own
   // rows and runs first; the fp32 kernels have a pass of its own.
   const bool dq_first = d->io_dtype != NXA_F32;

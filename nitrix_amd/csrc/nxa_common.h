@@ -532,6 +532,12 @@ __device__ __forceinline__ void dma16_buf(i32x4 rsrc, uint32_t voff, uint32_t ld
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
                :: "v"(voff), "s"(rsrc), "s"(m) : "m0");
 }
+// The same, marked non-temporal (streams read once).
+__device__ __forceinline__ void dma16_buf_nt(i32x4 rsrc, uint32_t voff, uint32_t lds) {
+  const uint32_t m = __builtin_amdgcn_readfirstlane(lds);
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen nt lds"
+               :: "v"(voff), "s"(rsrc), "s"(m) : "m0");
+}
 __device__ __forceinline__ void dma4_buf(i32x4 rsrc, uint32_t voff, uint32_t lds) {
   const uint32_t m = __builtin_amdgcn_readfirstlane(lds);
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds"

@@ -52,6 +52,16 @@ void launch_short(const Params& p, const ShortParams& sp, int io_dtype, ShortPar
 void launch_bias_pack(const Params& p, const ShortParams& sp, hipStream_t stream);
 void launch_dbias_slabs(const Params& p, const ShortParams& sp, void* out, const int64_t* str,
                         hipStream_t stream);
+// Few queries over many keys (nxa_split16.hip).
+constexpr int kSplitMaxQ = 64, kSplitMinK = 513;
+struct SplitParams {
+  int strips, splits;  // 32-query strips; key splits of each
+  float* part;         // [B H][strips][splits] partial results (splits > 1)
+};
+int split_count(int64_t strips, int Lk);  // strips over all (batch, head) pairs
+size_t split_part_bytes(int dp);
+void launch_fwd_split(const Params& p, const SplitParams& sp, int io_dtype, int dp,
+                      hipStream_t stream);
 void launch_rms_norm(const NormParams& p, int dtype, bool bwd, hipStream_t stream);
 int ssm_padded_states(int N);
 int ssm_lanes_per_channel(int NP);
