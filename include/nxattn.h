@@ -254,6 +254,26 @@ int nxa_ssm_bwd(int64_t nb, int32_t L, int32_t d, int32_t n, const float* x,
                 float* ddelta, float* dA, float* dB, float* dC, float* dD,
                 void* workspace, size_t workspace_bytes, void* stream);
 
+/* The same scan for up to 16 states with x, delta, B and C (and dx, ddelta,
+ * dB, dC) in `dtype` (nxa_dtype; A, D, y, dy, dA, dD and all arithmetic stay
+ * fp32), one kernel per direction plus one reduction: the whole sequence of a
+ * channel is walked inside one block, so there is no forward workspace.
+ * `state` (nxa_ssm_io_state_bytes, 16-byte aligned, its own layout: not
+ * interchangeable with nxa_ssm_fwd's) may be NULL in the forward when no backward follows; the
+ * backward's workspace (nxa_ssm_io_workspace_bytes, 256-byte aligned) holds
+ * per-channel-group partial sums of dB and dC.  Everything else as above;
+ * more states are NXA_E_UNSUPPORTED (nxa_ssm_fwd / nxa_ssm_bwd take them). */
+size_t nxa_ssm_io_state_bytes(int64_t nb, int32_t L, int32_t d, int32_t n);
+size_t nxa_ssm_io_workspace_bytes(int64_t nb, int32_t L, int32_t d, int32_t n);
+int nxa_ssm_io_fwd(int64_t nb, int32_t L, int32_t d, int32_t n, int32_t dtype, const void* x,
+                   const void* delta, const float* A, const void* B, const void* C,
+                   const float* D, float* y, float* state, void* stream);
+int nxa_ssm_io_bwd(int64_t nb, int32_t L, int32_t d, int32_t n, int32_t dtype, const void* x,
+                   const void* delta, const float* A, const void* B, const void* C,
+                   const float* D, const float* state, const float* dy, void* dx,
+                   void* ddelta, float* dA, void* dB, void* dC, float* dD,
+                   void* workspace, size_t workspace_bytes, void* stream);
+
 /* Message of the last failure on this thread ("" if none). */
 const char* nxa_last_error(void);
 

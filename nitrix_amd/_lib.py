@@ -63,6 +63,10 @@ EXPORTS = (
     'nxa_ssm_workspace_bytes',
     'nxa_ssm_fwd',
     'nxa_ssm_bwd',
+    'nxa_ssm_io_state_bytes',
+    'nxa_ssm_io_workspace_bytes',
+    'nxa_ssm_io_fwd',
+    'nxa_ssm_io_bwd',
     'nxa_last_error',
     'nxa_profile_enable',
     'nxa_profile_read',
@@ -162,6 +166,16 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.nxa_ssm_fwd.argtypes = [i64, i32, i32, i32] + [vp] * 9 + [ctypes.c_size_t, vp]
     lib.nxa_ssm_bwd.restype = ctypes.c_int
     lib.nxa_ssm_bwd.argtypes = [i64, i32, i32, i32] + [vp] * 15 + [ctypes.c_size_t, vp]
+    lib.nxa_ssm_io_state_bytes.restype = ctypes.c_size_t
+    lib.nxa_ssm_io_state_bytes.argtypes = [i64, i32, i32, i32]
+    lib.nxa_ssm_io_workspace_bytes.restype = ctypes.c_size_t
+    lib.nxa_ssm_io_workspace_bytes.argtypes = [i64, i32, i32, i32]
+    lib.nxa_ssm_io_fwd.restype = ctypes.c_int
+    lib.nxa_ssm_io_fwd.argtypes = [i64, i32, i32, i32, i32] + [vp] * 9
+    lib.nxa_ssm_io_bwd.restype = ctypes.c_int
+    lib.nxa_ssm_io_bwd.argtypes = (
+        [i64, i32, i32, i32, i32] + [vp] * 15 + [ctypes.c_size_t, vp]
+    )
     lib.nxa_last_error.restype = ctypes.c_char_p
     lib.nxa_last_error.argtypes = []
     lib.nxa_profile_enable.restype = ctypes.c_int

@@ -583,6 +583,71 @@ int check_ptrs(const void* const* ptrs, const char* const* names, int n) {
   return NXA_OK;
 }
 
+// Fused scan (nxa_scan.hip): up to 16 states, any of the three dtypes.
+int check_scan(int64_t nb, int32_t L, int32_t Dm, int32_t N, int32_t dtype) {
+  if (!known_dtype(dtype))
+    return fail(NXA_E_DTYPE, "dtype %d is not NXA_BF16, NXA_F16 or NXA_F32", dtype);
+  int rc = check_ssm(nb, L, Dm, N);
+  if (rc) return rc;
+  if (N > nxa::kScanMaxStates)
+    return fail(NXA_E_UNSUPPORTED, "fused selective scan: state dim n=%d exceeds %d", N,
+                nxa::kScanMaxStates);
+  // A chunk's rows, and the states of one step, are addressed with 32-bit
+  // byte offsets below 2^31; the backward's grid is one block per channel
+  // group of at least 8 channels.
+  if (Dm >= 1 << 24 || nb * (((int64_t)Dm + 3) / 4) >= (int64_t)1 << 30)
+    return fail(NXA_E_SHAPE, "fused selective scan: nb=%lld d=%d exceed the grid", (long long)nb,
+                Dm);
+  return NXA_OK;
+}
+
+struct ScanLayout {
+  int NP, ns, G;
+  size_t state, part, dA, dD;  // byte sizes
+};
+
+ScanLayout scan_layout(int64_t nb, int32_t L, int32_t Dm, int32_t N) {
+  ScanLayout s;
+  s.NP = nxa::scan_padded_states(N);
+  s.ns = (L + nxa::kSsmSub - 1) / nxa::kSsmSub;
+  s.G = nxa::scan_groups(Dm, s.NP, nxa::scan_bwd_states(nb, Dm, s.NP));
+  s.state = (size_t)nb * s.ns * s.NP * Dm * sizeof(float);
+  s.part = align256((size_t)s.G * nb * L * 2 * s.NP * sizeof(float));
+  s.dA = align256((size_t)nb * s.NP * Dm * sizeof(float));
+  s.dD = align256((size_t)nb * Dm * sizeof(float));
+  return s;
+}
+
+nxa::ScanParams scan_params(int64_t nb, int32_t L, int32_t Dm, int32_t N, const void* x,
+                            const void* delta, const float* A, const void* B, const void* C,
+                            const float* D, const float* state) {
+  nxa::ScanParams p{};
+  p.x = x;
+  p.delta = delta;
+  p.A = A;
+  p.B = B;
+  p.C = C;
+  p.D = D;
+  p.hs = const_cast<float*>(state);
+  p.nb = nb;
+  p.L = L;
+  p.Dm = Dm;
+  p.N = N;
+  p.ns = (L + nxa::kSsmSub - 1) / nxa::kSsmSub;
+  return p;
+}
+
+// Pointers of the fused scan: io of the dtype's size, f32 of 4 bytes.
+int check_scan_ptrs(int dtype, const void* const* io, int nio, const void* const* f32, int nf) {
+  for (int i = 0; i < nio + nf; ++i) {
+    const void* q = i < nio ? io[i] : f32[i - nio];
+    if (!q) return fail(NXA_E_ARG, "fused selective scan: a required pointer is NULL");
+    if (!aligned(q, i < nio ? esize(dtype) : 4))
+      return fail(NXA_E_LAYOUT, "fused selective scan: a pointer is not aligned to its element");
+  }
+  return NXA_OK;
+}
+
 // Validation shared by the forward entry points.
 int check_fwd(const nxa_desc* d, const void* q, const void* k, const void* v,
               const void* bias, const uint8_t* mask, const void* o) {
@@ -1133,6 +1198,68 @@ int nxa_ssm_bwd(int64_t nb, int32_t L, int32_t d, int32_t n, const float* x,
   p.ndblk_b = s.ndblk_b;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   return launch("ssm_bwd", st, [&] { nxa::launch_ssm(p, true, st); });
+}
+
+size_t nxa_ssm_io_state_bytes(int64_t nb, int32_t L, int32_t d, int32_t n) {
+  if (check_scan(nb, L, d, n, NXA_F32)) return 0;
+  return scan_layout(nb, L, d, n).state;
+}
+
+size_t nxa_ssm_io_workspace_bytes(int64_t nb, int32_t L, int32_t d, int32_t n) {
+  if (check_scan(nb, L, d, n, NXA_F32)) return 0;
+  const ScanLayout s = scan_layout(nb, L, d, n);
+  return s.part + s.dA + s.dD;
+}
+
+int nxa_ssm_io_fwd(int64_t nb, int32_t L, int32_t d, int32_t n, int32_t dtype, const void* x,
+                   const void* delta, const float* A, const void* B, const void* C,
+                   const float* D, float* y, float* state, void* stream) {
+  int rc = check_scan(nb, L, d, n, dtype);
+  if (rc) return rc;
+  const void* io[4] = {x, delta, B, C};
+  const void* f32[2] = {A, y};
+  if ((rc = check_scan_ptrs(dtype, io, 4, f32, 2))) return rc;
+  if ((D && !aligned(D, 4)) || (state && !aligned(state, 16)))
+    return fail(NXA_E_LAYOUT,
+                "fused selective scan: D not 4-byte or state not 16-byte aligned");
+  nxa::ScanParams p = scan_params(nb, L, d, n, x, delta, A, B, C, D, state);
+  p.y = y;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  return launch("ssm_fwd", st, [&] { nxa::launch_scan(p, dtype, false, st); });
+}
+
+int nxa_ssm_io_bwd(int64_t nb, int32_t L, int32_t d, int32_t n, int32_t dtype, const void* x,
+                   const void* delta, const float* A, const void* B, const void* C,
+                   const float* D, const float* state, const float* dy, void* dx, void* ddelta,
+                   float* dA, void* dB, void* dC, float* dD, void* workspace,
+                   size_t workspace_bytes, void* stream) {
+  int rc = check_scan(nb, L, d, n, dtype);
+  if (rc) return rc;
+  const void* io[8] = {x, delta, B, C, dx, ddelta, dB, dC};
+  const void* f32[4] = {A, state, dy, dA};
+  if ((rc = check_scan_ptrs(dtype, io, 8, f32, 4))) return rc;
+  if ((D && !aligned(D, 4)) || (dD && !aligned(dD, 4)) || !aligned(state, 16))
+    return fail(NXA_E_LAYOUT,
+                "fused selective scan: D / dD not 4-byte or state not 16-byte aligned");
+  const ScanLayout s = scan_layout(nb, L, d, n);
+  if (!workspace || workspace_bytes < s.part + s.dA + s.dD || !aligned(workspace, 256))
+    return fail(NXA_E_WORKSPACE,
+                "fused selective scan: workspace needs %zu bytes, 256-byte aligned",
+                s.part + s.dA + s.dD);
+  nxa::ScanParams p = scan_params(nb, L, d, n, x, delta, A, B, C, D, state);
+  p.dy = dy;
+  p.dx = dx;
+  p.ddelta = ddelta;
+  p.dA = dA;
+  p.dB = dB;
+  p.dC = dC;
+  p.dD = D ? dD : nullptr;
+  char* ws = static_cast<char*>(workspace);
+  p.part = reinterpret_cast<float*>(ws);
+  p.dApart = reinterpret_cast<float*>(ws + s.part);
+  p.dDpart = reinterpret_cast<float*>(ws + s.part + s.dA);
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  return launch("ssm_bwd", st, [&] { nxa::launch_scan(p, dtype, true, st); });
 }
 
 int nxa_profile_enable(int on) {

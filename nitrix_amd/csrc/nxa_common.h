@@ -210,6 +210,23 @@ struct SsmParams {
   int ndblk_b;    // channel blocks of the backward chunk pass (lanes per channel > 1)
 };
 
+// Parameter block of the fused scan kernels (nxa_scan.hip; N <= 16, NP = 8
+// or 16 padded states).
+struct ScanParams {
+  const void *x, *delta, *B, *C;  // [nb, L, Dm] and [nb, L, N], one dtype
+  const float *A, *D;             // [Dm, N], [Dm] (may be null)
+  float* y;                       // [nb, L, Dm]
+  float* hs;                      // [nb][ns][Dm][NP] state entering every 8 steps (may be null)
+  const float* dy;
+  void *dx, *ddelta, *dB, *dC;    // as x, delta, B, C
+  float *dA, *dD;                 // dD may be null
+  float* part;                    // [G][nb][L][2 NP] dB / dC partial rows
+  float *dApart, *dDpart;         // [nb][NP][Dm], [nb][Dm]
+  int64_t nb, L;
+  int Dm, N, ns;
+  int G;                          // channel groups (set by the launcher)
+};
+
 // How the 16-bit forward adds the bias (chosen on the host).
 //  * kFbRow  / kFbTile: the bias enters the score accumulator through MFMA
 //    products bias^T x diag(1/scale) (1/scale split into two terms of the

@@ -70,6 +70,12 @@ constexpr int kSsmSub = 8;      // steps per saved sub-chunk state
 constexpr int kSsmDadGroups = 16;  // row groups of the dA / dD reduction
 constexpr int kSsmBlock = 256;  // channels per block of the selective scan
 void launch_ssm(const SsmParams& p, bool bwd, hipStream_t stream);
+// Fused scan (nxa_scan.hip).
+constexpr int kScanMaxStates = 16;
+int scan_padded_states(int N);
+int scan_groups(int Dm, int NP, int npl);  // channel groups with npl states a lane
+int scan_bwd_states(int64_t nb, int Dm, int NP);  // states a lane in the backward
+void launch_scan(const ScanParams& p, int dtype, bool bwd, hipStream_t stream);
 // One chunk of the dbias reduction over broadcast batch / head axes.
 struct DbiasReduce {
   const float* part;  // [nbh, LQ, Lk] fp32 partials of pairs bh0 .. bh0 + nbh - 1

@@ -15,10 +15,13 @@ reference's public call signature and layering:
   in stock tensor ops, with its ``'sequential'``, ``'associative'`` and
   ``'chunked'`` drivers.
 
-The fused kernels compute in float32.  bfloat16 / float16 inputs are upcast
-at the boundary and the output cast back, as the reference's float32
-accumulation rule does (``_reference.py:255-281``); float64 is declined (a
-loud fallback to the reference engine).
+The fused kernels compute in float32, as the reference's float32
+accumulation rule asks (``_reference.py:255-281``).  Up to 16 states
+(``nxa_ssm_io_fwd`` / ``nxa_ssm_io_bwd``) bfloat16 / float16 x, delta, B and C
+of one dtype are read, and their gradients written, in that dtype; other
+mixes and more states (``nxa_ssm_fwd`` / ``nxa_ssm_bwd``) are upcast at the
+boundary and the results cast back.  float64 is declined (a loud fallback to
+the reference engine).
 """
 
 from __future__ import annotations
@@ -46,8 +49,13 @@ __all__ = [
 ]
 
 _DRIVERS = ('auto', 'sequential', 'associative', 'chunked')
-_HIP_DTYPES = (torch.float32, torch.bfloat16, torch.float16)
+_HIP_DTYPES = {
+    torch.float32: _lib.NXA_F32,
+    torch.bfloat16: _lib.NXA_BF16,
+    torch.float16: _lib.NXA_F16,
+}
 _MAX_STATES = 32
+_MAX_IO_STATES = 16  # nxa_ssm_io_fwd / nxa_ssm_io_bwd
 
 
 def _validate(x, delta, A, B, C, D) -> None:
@@ -227,10 +235,27 @@ def _unbroadcast(g: torch.Tensor, shape) -> torch.Tensor:
     return g
 
 
-class _ScanPrep:
-    """float32 [nb, l, d] / [nb, l, n] views and the extents of one call."""
+def _takes_fused(nb: int, length: int, d: int, n: int, train: bool) -> bool:
+    """Whether ``nxa_ssm_io_*`` take the call, else ``nxa_ssm_*``.
 
-    def __init__(self, x, delta, A, B, C, D):
+    They hold up to 16 states and 32-bit offsets.  One block walks the whole
+    sequence of its channels, so a training step on a long sequence of few
+    channels (which leaves most CUs idle) takes 47.5 ns a step (batch 1, d
+    512, n 16, L 8192: 399 us), where the chunk-parallel kernels take about
+    70 us + 18 ns a step + 1.3 us per million state steps (290 us): they keep
+    L > 2400 + 4e-5 (state steps).  At L 2048 the fused kernels lead (109 us
+    against 133), with more channels too (batch 4: 598 against 725)."""
+    if n > _MAX_IO_STATES or d >= 1 << 24 or nb * (d // 4 + 1) >= 1 << 30:
+        return False
+    states = 8 if n <= 8 else 16
+    return not train or length <= 2400 + 4e-5 * nb * length * d * states
+
+
+class _ScanPrep:
+    """Contiguous [nb, l, d] / [nb, l, n] views (in the scan's dtype) and the
+    extents of one call."""
+
+    def __init__(self, x, delta, A, B, C, D, train):
         f32 = torch.float32
         *batch, length, d = x.shape
         self.batch = tuple(batch)
@@ -242,9 +267,17 @@ class _ScanPrep:
         self.dtypes = [t.dtype for t in (x, delta, A, B, C)]
         self.D_dtype = None if D is None else D.dtype
         bn = self.batch + (length, self.n)
+        # The dtype the kernels read x, delta, B and C in (float32 also where
+        # gradients of a broadcast B or C are summed over their copies).
+        self.fused = _takes_fused(self.nb, length, d, self.n, train)
+        one = (
+            x.dtype == delta.dtype == B.dtype == C.dtype
+            and tuple(B.shape) == tuple(C.shape) == bn
+        )
+        self.scan = x.dtype if self.fused and one and x.dtype in _HIP_DTYPES else f32
 
         def flat(t, shape, last):
-            return t.to(f32).expand(shape).reshape(self.nb, length, last).contiguous()
+            return t.to(self.scan).expand(shape).reshape(self.nb, length, last).contiguous()
 
         self.x = flat(x, self.batch + (length, d), d)
         self.delta = flat(delta, self.batch + (length, d), d)
@@ -272,6 +305,18 @@ def _scan_forward(prep: _ScanPrep, keep_state: bool):
     lib = _lib.lib()
     y = torch.empty((prep.nb, prep.length, prep.d), dtype=torch.float32, device=prep.device)
     state = None
+    if prep.fused:
+        if keep_state:
+            nbytes = lib.nxa_ssm_io_state_bytes(*prep.dims())
+            state = torch.empty(nbytes // 4, dtype=torch.float32, device=prep.device)
+        _lib.check(
+            lib.nxa_ssm_io_fwd(
+                *prep.dims(), _HIP_DTYPES[prep.scan],
+                _p(prep.x), _p(prep.delta), _p(prep.A), _p(prep.B), _p(prep.C), _p(prep.D),
+                _p(y), _p(state), prep.stream(),
+            )
+        )
+        return y, state
     if keep_state:
         nbytes = lib.nxa_ssm_state_bytes(*prep.dims())
         state = torch.empty(nbytes // 4, dtype=torch.float32, device=prep.device)
@@ -296,6 +341,18 @@ def _scan_backward(prep: _ScanPrep, state: torch.Tensor, dy: torch.Tensor):
     dB = torch.empty_like(prep.B)
     dC = torch.empty_like(prep.C)
     dD = None if prep.D is None else torch.empty_like(prep.D)
+    if prep.fused:
+        nbytes = lib.nxa_ssm_io_workspace_bytes(*prep.dims())
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=prep.device)
+        _lib.check(
+            lib.nxa_ssm_io_bwd(
+                *prep.dims(), _HIP_DTYPES[prep.scan],
+                _p(prep.x), _p(prep.delta), _p(prep.A), _p(prep.B), _p(prep.C), _p(prep.D),
+                _p(state), _p(dy), _p(dx), _p(ddelta), _p(dA), _p(dB), _p(dC), _p(dD),
+                _p(ws), ws.numel(), prep.stream(),
+            )
+        )
+        return dx, ddelta, dA, dB, dC, dD
     ws = prep.workspace(1)
     _lib.check(
         lib.nxa_ssm_bwd(
@@ -311,16 +368,16 @@ def _scan_backward(prep: _ScanPrep, state: torch.Tensor, dy: torch.Tensor):
 class _ScanHip(torch.autograd.Function):
     """Fused forward, recompute-adjoint fused backward.
 
-    The fp32 views the kernels read (which alias the caller's tensors when
-    those are already contiguous fp32) and the saved sub-chunk states are
+    The views the kernels read (which alias the caller's tensors when those
+    are already contiguous in the scan's dtype) and the saved sub-chunk states are
     kept with ``save_for_backward``, so an in-place change of an input
     between forward and backward raises torch's version-counter error; the
     backward is not itself differentiable."""
 
     @staticmethod
     def forward(ctx, x, delta, A, B, C, D):
-        prep = _ScanPrep(x, delta, A, B, C, D)
         keep = any(ctx.needs_input_grad)
+        prep = _ScanPrep(x, delta, A, B, C, D, keep)
         y, state = _scan_forward(prep, keep)
         if keep:
             ctx.save_for_backward(prep.x, prep.delta, prep.A, prep.B, prep.C, prep.D, state)

@@ -1,0 +1,86 @@
+"""Parity of the fused scan kernels (up to 16 states, x, delta, B and C in
+fp32, bf16 or fp16) against the float64 oracle at the edges of their chunks,
+channel groups and dispatch: lengths around 8 and the steps of one
+iteration, channel counts around a group, state counts around the padding,
+batches that select each states-per-lane variant, and the first shapes that
+stay with the chunk-parallel kernels."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import ssm as S
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = {'f32': torch.float32, 'bf16': torch.bfloat16, 'f16': torch.float16}
+# Relative 2-norm of the gradients written in the scan's dtype: its rounding.
+TOL = {'f32': 2e-6, 'bf16': 4e-3, 'f16': 5e-4}
+
+
+def _check(name, nb, length, d, n, with_d=True, seed=0):
+    dtype, dev = DTYPES[name], torch.device('cuda:0')
+    g = torch.Generator().manual_seed(seed)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g)
+
+    x, B, C = rnd(nb, length, d), rnd(nb, length, n), rnd(nb, length, n)
+    delta = 0.01 + 0.3 * torch.sigmoid(rnd(nb, length, d))
+    io = [t.to(dtype) for t in (x, delta, B, C)]
+    A = -(0.2 + rnd(d, n).abs())
+    D = rnd(d) if with_d else None
+    dy = rnd(nb, length, d)
+    from nitrix_amd import selective_scan
+
+    leaves = [t.to(dev).requires_grad_(True) for t in (io[0], io[1], A, io[2], io[3])]
+    if with_d:
+        leaves.append(D.to(dev).requires_grad_(True))
+    print(f'[case] scan {name} b{nb} L{length} d{d} n{n} D={with_d}', flush=True)
+    y = selective_scan(*leaves, backend='hip')
+    with torch.no_grad():
+        y0 = selective_scan(*[t.detach() for t in leaves], backend='hip')
+    grads = torch.autograd.grad(y, leaves, dy.to(dev))
+    a64 = [t.double().numpy() for t in (io[0], io[1], A, io[2], io[3])]
+    a64.append(D.double().numpy() if with_d else None)
+    want = [S.selective_scan(*a64)] + [w for w in S.selective_scan_vjp(*a64, dy.double().numpy())
+                                       if w is not None]
+    assert y.dtype == y0.dtype == torch.float32
+    for i, (got, ref) in enumerate(zip([y, *grads], want)):
+        got = got.detach().double().cpu().numpy()
+        tol = TOL['f32'] if i == 0 or i == 3 or i == 6 else TOL[name]
+        # (dA is exactly zero for a single step: both sides then are)
+        assert np.linalg.norm(got - ref) <= tol * np.linalg.norm(ref), i
+    err = np.linalg.norm(y0.double().cpu().numpy() - want[0]) / np.linalg.norm(want[0])
+    assert err <= TOL['f32'], err
+
+
+@pytest.mark.parametrize('name', ['f32', 'bf16', 'f16'])
+@pytest.mark.parametrize('nb, length, d, n', [
+    (1, 1, 1, 1), (2, 7, 5, 3), (1, 8, 16, 8), (3, 9, 17, 9), (1, 129, 33, 16), (2, 257, 31, 5),
+    (1, 1025, 8, 16), (700, 20, 9, 16), (300, 33, 40, 8),
+])
+def test_chunks_groups_and_states(name, nb, length, d, n):
+    _check(name, nb, length, d, n, with_d=n % 2 == 0, seed=length)
+
+
+@pytest.mark.parametrize('name, length', [('f32', 2400), ('bf16', 2403), ('f32', 2600)])
+def test_both_sides_of_the_long_sequence_rule(name, length):
+    _check(name, 1, length, 12, 4, seed=length)
+
+
+def test_seventeen_states_and_mixed_dtypes():
+    _check('bf16', 2, 100, 20, 17)
+    dev = torch.device('cuda:0')
+    g = torch.Generator().manual_seed(1)
+    x, B, C = (torch.randn(2, 50, k, generator=g) for k in (24, 8, 8))
+    delta = 0.1 * torch.rand(2, 50, 24, generator=g)
+    A = -torch.rand(24, 8, generator=g)
+    from nitrix_amd import selective_scan
+
+    xb = x.to(torch.bfloat16)
+    y = selective_scan(*[t.to(dev) for t in (xb, delta, A, B, C)], backend='hip')
+    ref = S.selective_scan(*[t.double().numpy() for t in (xb, delta, A, B, C)], None)
+    assert np.linalg.norm(y.double().cpu().numpy() - ref) / np.linalg.norm(ref) <= 2e-6
