@@ -65,22 +65,21 @@ PEAK_HBM_GBS = 8000.0
 # TRAFFIC_SRC is the fingerprint (_src_fingerprint) of the attention kernel
 # sources the passes ran; when the sources differ, the figure describes other
 # kernels and is reported as stale (traffic null, the old figure beside it).
-TRAFFIC_SRC = '31b32cd5e083de76'
+TRAFFIC_SRC = '3424b6891ab6ff98'
 MEASURED_TRAFFIC = {
-    'c1': ('fwd', 6102721),
-    'c2': ('dkdv', 910444756),
-    'c3': ('dkdv', 1619918515),
-    'c4': ('fwd', 4431184901),
-    'c5': ('dkdv', 706542360),
+    'c1': ('fwd', 6102699),
+    'c2': ('dkdv', 910863461),
+    'c3': ('dkdv', 1619817728),
+    'c4': ('fwd', 4431318736),
+    'c5': ('dkdv', 706809013),
 }
-# VALU instructions (wave64) of the selective scan's backward pass (all five
+# VALU instructions (wave64) of the selective scan's backward pass (both
 # kernels) per step at the ssm configuration, transcendental instructions
-# weighted 4: the
-# rocprofv3 SQ_INSTS_VALU / SQ_INSTS_VALU_TRANS_F32 counts of its kernels in
+# weighted 4: the rocprofv3 SQ_INSTS_VALU / SQ_INSTS_VALU_TRANS_F32 counts of its kernels in
 # profiles/selective_scan_valu_counters.md.
-SSM_BWD_VALU_WAVE_INSTS = 2.5654e8
-# Fingerprint of nxa_ssm.hip + nxa_common.h when the counts were taken.
-SSM_VALU_SRC = 'fa3803c37f913189'
+SSM_BWD_VALU_WAVE_INSTS = 1.7965e8
+# Fingerprint of nxa_scan.hip + nxa_common.h when the counts were taken.
+SSM_VALU_SRC = '7f743280a8be0215'
 SSM_VALU_SOURCE = 'profiles/selective_scan_valu_counters.md (rocprofv3 SQ_INSTS_VALU, SQ_INSTS_VALU_TRANS_F32)'
 PEAK_VALU_TLANEOPS = 256 * 4 * 32 * 2.4e9 / 1e12  # 78.6 T lane-instructions/s
 TRAFFIC_SOURCE = 'profiles/attention_hbm_traffic_c1_c5.md (rocprofv3 FETCH_SIZE x2 + WRITE_SIZE x1)'
@@ -185,7 +184,7 @@ def _sparse_blocks(L):
 ATTN_SOURCES = ('nxa_common.h', 'nxa_launch.h', 'nxa_fwd16.h', 'nxa_bwd16.h', 'nxa_fwd16.hip',
                 'nxa_fwd16_wide.hip', 'nxa_bwd16.hip', 'nxa_bwd16_wide.hip', 'nxa_fwd.hip',
                 'nxa_bwd.hip', 'nxa_attn32.hip', 'nxa_capi.hip', 'nxa_norm.hip')
-SSM_SOURCES = ('nxa_common.h', 'nxa_ssm.hip')
+SSM_SOURCES = ('nxa_common.h', 'nxa_scan.hip')
 
 
 def _src_fingerprint(names) -> str:
@@ -498,9 +497,9 @@ def _bench_ssm(args, torch) -> int:
     _lib.profile_reset()
     assert all(torch.isfinite(t.grad).all() for t in leaves), 'non-finite gradient'
     fwd_b, bwd_b = _ssm_bytes(Bn, L, Dm, N)
-    # The backward pass (five kernels) dominates and is bound by VALU issue
+    # The backward pass (two kernels) dominates and is bound by VALU issue
     # (one exponential and a few fp32 operations per state step; its
-    # compulsory bytes move at ~10 % of HBM bandwidth).  Its VALU work per
+    # compulsory bytes move at ~17 % of HBM bandwidth).  Its VALU work per
     # step is the counted instructions of its kernels (transcendentals
     # weighted 4, quarter rate) times 64 lanes, over its measured duration,
     # against 256 CUs x 4 SIMDs x 32 lanes x 2.4 GHz (the published
@@ -510,7 +509,7 @@ def _bench_ssm(args, torch) -> int:
     achieved = lane_ops / bwd_s / 1e12
     src = _src_fingerprint(SSM_SOURCES)
     roofline = {
-        'kernel': 'ssm_bwd (backward pass: local, carry, chunk, two reductions)',
+        'kernel': 'ssm_bwd (backward pass: the scan and the reduction of dB, dC, dA, dD)',
         'bound': 'valu',
         'achieved': round(achieved, 3),
         'peak': PEAK_VALU_TLANEOPS,
