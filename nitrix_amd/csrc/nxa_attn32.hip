@@ -566,17 +566,21 @@ enum : int { kF32Dv = 1, kF32Dk = 2, kF32Both = 3 };
 // stationary rows and both accumulator sets do not fit one wave's
 // registers: two launches, OUT = kF32Dv (K stationary; S, P, dV) and then
 // kF32Dk (K, V stationary; S, dP, dS, dK, dbias), over 32-query tiles.
+// SPLIT: the four waves share 32 keys and take every fourth 32-query tile, in
+// a stage of their own; their sums are added in LDS in a fixed order.
 // ---------------------------------------------------------------------------
-template <int DP, bool CAUSAL, int OUT = kF32Both>
-__global__ __launch_bounds__(256, 1) void dkdv32_kernel(const Params p) {
+template <int DP, bool CAUSAL, int OUT = kF32Both, bool SPLIT = false>
+__global__ __launch_bounds__(256, SPLIT ? 2 : 1) void dkdv32_kernel(const Params p) {
   constexpr bool DV = OUT & kF32Dv, DK = OUT & kF32Dk;
   static_assert(OUT == kF32Both || DP > 128, "split launches are for head dim 256");
-  constexpr int BNK = 128, BQ = OUT == kF32Both ? 64 : 32, NQB = BQ / 32;
+  static_assert(!SPLIT || (OUT == kF32Both && DP == 64), "the merge is of dV and dK at head dim 64");
+  constexpr int NW = SPLIT ? 1 : 4;  // waves that share a tile
+  constexpr int BNK = 32 * NW, BQ = OUT == kF32Both && !SPLIT ? 64 : 32, NQB = BQ / 32;
   constexpr int NC = DP / 8, NDB = DP / 32;
   constexpr int TILE = BQ * DP * 4;
   constexpr int STAGE = 2 * TILE + 2 * BQ * 4;  // Q, dO, -lse log2(e), -delta
-  using S = F32Stream<DP, 4, BQ, (DP > 128)>;
-  __shared__ __attribute__((aligned(16))) char smem[2 * STAGE];
+  using S = F32Stream<DP, NW, BQ, (DP > 128)>;
+  __shared__ __attribute__((aligned(16))) char smem[(SPLIT ? 4 : 2) * STAGE];
   __shared__ uint32_t lst[kF32MaxTiles];
 
   const int vid = xcd_remap(blockIdx.x, p.nbh, p.nkt);
@@ -587,7 +591,8 @@ __global__ __launch_bounds__(256, 1) void dkdv32_kernel(const Params p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5, c32 = lane & 31;
   const int kblk0 = kt * BNK;
-  const int kw0 = kblk0 + wave * 32;
+  const int cw = SPLIT ? 0 : wave;  // wave of those that share a tile
+  const int kw0 = kblk0 + cw * 32;
   const int key = kw0 + c32;
   const bool kok = key < p.Lk;
   const int kc = kok ? key : p.Lk - 1;
@@ -626,15 +631,15 @@ __global__ __launch_bounds__(256, 1) void dkdv32_kernel(const Params p) {
   float colsum = 0.f;
 
   S qs, ds_;
-  qs.init(p.q_str[2], p.D, wave, lane);
-  ds_.init(p.o_str[2], p.Dv, wave, lane);
+  qs.init(p.q_str[2], p.D, cw, lane);
+  ds_.init(p.o_str[2], p.Dv, cw, lane);
   F32Offsets<DP> lo;
   lo.init(g, c32);
   const uint32_t lds0 = lds_offset(smem);
 
   // Copies of active tile i (empty ranges past the list) into stage st:
-  // CNT Q and CNT dO copies, and BQ / 4 rows of -lse log2(e) and -delta per
-  // wave (lanes 0 .. BQ / 4 - 1).
+  // CNT Q and CNT dO copies, and BQ / NW rows of -lse log2(e) and -delta per
+  // wave (lanes 0 .. BQ / NW - 1).
   auto issue = [&](int i, int st) NXA_INLINE {
     const int t = i < n ? (int)(lst[i] & 0xffff) : nq;
     const int q0 = t * BQ;
@@ -643,16 +648,16 @@ __global__ __launch_bounds__(256, 1) void dkdv32_kernel(const Params p) {
     const i32x4 ro = tile_rsrc<BQ>(dop, p.o_str[2], q0, p.Lq, p.Dv);
 #pragma unroll
     for (int m = 0; m < S::CNT; ++m) {
-      qs.issue(rq, at, m, wave);
-      ds_.issue(ro, at + TILE, m, wave);
+      qs.issue(rq, at, m, cw);
+      ds_.issue(ro, at + TILE, m, cw);
     }
     const int rows = max(min(BQ, p.Lq - q0), 0);
-    constexpr int RW = BQ / 4;  // row values per wave
+    constexpr int RW = BQ / NW;  // row values per wave
     if (lane < RW) {
-      dma4_buf(make_rsrc(nlp + min(q0, p.Lq), (uint32_t)rows * 4u), 4u * (RW * wave + lane),
-               at + 2 * TILE + 4 * RW * wave);
-      dma4_buf(make_rsrc(ndp + min(q0, p.Lq), (uint32_t)rows * 4u), 4u * (RW * wave + lane),
-               at + 2 * TILE + BQ * 4 + 4 * RW * wave);
+      dma4_buf(make_rsrc(nlp + min(q0, p.Lq), (uint32_t)rows * 4u), 4u * (RW * cw + lane),
+               at + 2 * TILE + 4 * RW * cw);
+      dma4_buf(make_rsrc(ndp + min(q0, p.Lq), (uint32_t)rows * 4u), 4u * (RW * cw + lane),
+               at + 2 * TILE + BQ * 4 + 4 * RW * cw);
     }
   };
   constexpr int CPT = 2 * S::CNT + 2;  // copies per wave per tile
@@ -662,7 +667,7 @@ __global__ __launch_bounds__(256, 1) void dkdv32_kernel(const Params p) {
   const int64_t dbbase = b * p.dbias_str[0] + h * p.dbias_str[1] + key - p.dbias_off;
   const bool full_db = p.dbias_mode == kDbiasFull;
 
-  if (n > 0) issue(0, 0);
+  if (!SPLIT && n > 0) issue(0, 0);
   if (DK && full_db && kok) {
     // A full dbias gets zeros where no query of a tile keeps this key block.
     int li = 0;
@@ -671,25 +676,34 @@ __global__ __launch_bounds__(256, 1) void dkdv32_kernel(const Params p) {
         ++li;
         continue;
       }
+      if (SPLIT && (t & 3) != wave) continue;
       for (int q = t * BQ; q < min(t * BQ + BQ, p.Lq); ++q)
         store_db32(p, dbbase + (int64_t)q * p.dbias_str[2], 0.f);
     }
   }
-  __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-  __syncthreads();
-  for (int i = 0; i < n; ++i) {
-    const int st = i & 1;
+  if constexpr (!SPLIT) {
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    __syncthreads();
+  }
+  for (int i = SPLIT ? wave : 0; i < n; i += SPLIT ? 4 : 1) {
+    const int st = SPLIT ? wave : i & 1;
     const uint32_t at = lds0 + st * STAGE;
     const int t = (int)(lst[i] & 0xffff), cls = (int)(lst[i] >> 16);
     const int q0 = t * BQ;
-    issue(i + 1, st ^ 1);
+    if constexpr (SPLIT) {
+      // Only this wave reads its stage: its own wait publishes the copies.
+      issue(i, st);
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    } else {
+      issue(i + 1, st ^ 1);
+    }
 
     // S = Q K^T and dP = dO V^T.  Both outputs: acc[0..1] = S of query
     // blocks 0, 1, acc[2..3] = dP.  dK: acc[0] = S, acc[1] = dP of the one
     // 32-query block.  dV: S over the low and the high half of the head
     // dim, summed after.  The A fragments of step c + 1 are read while the
-    // MFMAs of step c run.
-    constexpr int NA = OUT == kF32Both ? 4 : 2;
+    // MFMAs of step c run.  (Split: as dK, one 32-query block.)
+    constexpr int NA = 2 * NQB;
     constexpr int NSTEP = OUT == kF32Dv ? NC / 2 : NC;
     f32x16 acc[NA];
 #pragma unroll
@@ -699,12 +713,12 @@ __global__ __launch_bounds__(256, 1) void dkdv32_kernel(const Params p) {
     {
       f32x4 a[2][NA], bq[NA];
       auto rd = [&](f32x4* x, int c) NXA_INLINE {
-        if constexpr (OUT == kF32Both) {
+        if constexpr (NQB == 2) {
           x[0] = lo.row(at, 0, c);
           x[1] = lo.row(at, 1, c);
           x[2] = lo.row(at + TILE, 0, c);
           x[3] = lo.row(at + TILE, 1, c);
-        } else if constexpr (OUT == kF32Dk) {
+        } else if constexpr (DK) {
           x[0] = lo.row(at, 0, c);
           x[1] = lo.row(at + TILE, 0, c);
         } else {
@@ -716,10 +730,10 @@ __global__ __launch_bounds__(256, 1) void dkdv32_kernel(const Params p) {
 #pragma unroll
       for (int c = 0; c < NSTEP; ++c) {
         if (c + 1 < NSTEP) rd(a[(c + 1) & 1], c + 1);
-        if constexpr (OUT == kF32Both) {
+        if constexpr (NQB == 2) {
           bq[0] = bq[1] = kf[c];
           bq[2] = bq[3] = vf[c];
-        } else if constexpr (OUT == kF32Dk) {
+        } else if constexpr (DK) {
           bq[0] = kf[c];
           bq[1] = vf[c];
         } else {
@@ -815,7 +829,7 @@ __global__ __launch_bounds__(256, 1) void dkdv32_kernel(const Params p) {
     }
 #pragma unroll
     for (int hb = 0; hb < (OUT == kF32Both ? NDB : 0); hb += 2) {
-      constexpr int NA = NDB >= 2 ? 4 : 2;
+      constexpr int NA = NDB >= 2 ? 4 : 2, NS = 4 * NQB;
       f32x16 o[NA];
 #pragma unroll
       for (int u = 0; u < NA / 2; ++u) {
@@ -833,8 +847,8 @@ __global__ __launch_bounds__(256, 1) void dkdv32_kernel(const Params p) {
       };
       rd(a[0], 0);
 #pragma unroll
-      for (int step = 0; step < 8; ++step) {
-        if (step + 1 < 8) rd(a[(step + 1) & 1], step + 1);
+      for (int step = 0; step < NS; ++step) {
+        if (step + 1 < NS) rd(a[(step + 1) & 1], step + 1);
         const int j = step >> 2, f = step & 3;
 #pragma unroll
         for (int u = 0; u < NA / 2; ++u) {
@@ -845,7 +859,7 @@ __global__ __launch_bounds__(256, 1) void dkdv32_kernel(const Params p) {
       }
       __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 8 * NA, 0);
 #pragma unroll
-      for (int step = 0; step < 6; ++step) {
+      for (int step = 0; step + 2 < NS; ++step) {
         __builtin_amdgcn_sched_group_barrier(kSchedMfma, 4 * NA, 0);
         __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 4 * NA, 0);
       }
@@ -857,12 +871,56 @@ __global__ __launch_bounds__(256, 1) void dkdv32_kernel(const Params p) {
       }
     }
 
-    // Tile i + 1 is resident, and every wave is done with stage st, before
-    // the next iteration.
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-    __syncthreads();
+    if constexpr (SPLIT) {
+      // The next copies overwrite the stage the products just read.
+      __builtin_amdgcn_s_waitcnt(lgkmcnt_imm(0));
+    } else {
+      // Tile i + 1 is resident, and every wave is done with stage st, before
+      // the next iteration.
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+      __syncthreads();
+    }
   }
   static_assert(CPT <= 63, "copies per tile fit the vmcnt counter");
+
+  if constexpr (SPLIT) {
+    // Sums of the four waves, [field][wave][lane] floats; wave w adds and
+    // stores block w / 2 of dV (even w) or dK (odd w).
+    __syncthreads();
+    float* ms = reinterpret_cast<float*>(smem);
+    constexpr int F = 2 * NDB * 16 + 1;
+    static_assert(F * 4 * 64 * 4 <= 4 * STAGE && NDB == 2, "the sums fit the stages");
+    auto slot = [&](int f, int w) -> float& { return ms[(f * 4 + w) * 64 + lane]; };
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        slot((2 * db) * 16 + r, wave) = dv[db][r];
+        slot((2 * db + 1) * 16 + r, wave) = dk[db][r];
+      }
+    slot(F - 1, wave) = colsum;
+    __syncthreads();
+    auto total = [&](int f) { return (slot(f, 0) + slot(f, 1)) + (slot(f, 2) + slot(f, 3)); };
+    f32x16 o;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[r] = total(wave * 16 + r);
+    if (kok) {
+      const bool is_k = wave & 1;
+      float* op = is_k ? (float*)p.dk + b * p.k_str[0] + h * p.k_str[1] + (int64_t)key * p.k_str[2]
+                       : (float*)p.dv + b * p.v_str[0] + h * p.v_str[1] + (int64_t)key * p.v_str[2];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int d0 = (wave >> 1) * 32 + 8 * c + 4 * g;
+        if (d0 < (is_k ? p.D : p.Dv)) store4(op + d0, o, 4 * c, is_k ? p.scale : 1.0f);
+      }
+    }
+    if (p.dbias_mode == kDbiasColsum && wave == 0) {
+      const float cs = total(F - 1);
+      const float tot = cs + shfl_xor32(cs);
+      if (kok && g == 0) store_db32(p, dbbase, tot);
+    }
+    return;
+  }
 
   if (kok) {
     float* dkp = (float*)p.dk + b * p.k_str[0] + h * p.k_str[1] + (int64_t)key * p.k_str[2];
@@ -887,14 +945,16 @@ __global__ __launch_bounds__(256, 1) void dkdv32_kernel(const Params p) {
 // 256, so that two stages of K and V fit the LDS).  A wave holds its
 // queries' Q and dO stationary and forms S^T = K Q^T and dP^T = V dO^T with
 // the query on the lane's column, so dS^T feeds dQ^T += K^T dS^T.
+// SPLIT as in dK / dV: 32 queries a block, every fourth 32-key tile a wave.
 // ---------------------------------------------------------------------------
-template <int DP, bool CAUSAL>
-__global__ __launch_bounds__(256, 1) void dq32_kernel(const Params p) {
-  constexpr int BM = 128, BN = DP > 128 ? 32 : 64, NKB = BN / 32, NC = DP / 8, NDB = DP / 32;
+template <int DP, bool CAUSAL, bool SPLIT = false>
+__global__ __launch_bounds__(256, SPLIT ? 2 : 1) void dq32_kernel(const Params p) {
+  constexpr int NW = SPLIT ? 1 : 4;  // waves that share a tile
+  constexpr int BM = 32 * NW, BN = DP > 128 || SPLIT ? 32 : 64, NKB = BN / 32, NC = DP / 8, NDB = DP / 32;
   constexpr int TILE = BN * DP * 4;
   constexpr int STAGE = 2 * TILE;  // K, V
-  using S = F32Stream<DP, 4, BN, (DP > 128)>;
-  __shared__ __attribute__((aligned(16))) char smem[2 * STAGE];
+  using S = F32Stream<DP, NW, BN, (DP > 128)>;
+  __shared__ __attribute__((aligned(16))) char smem[(SPLIT ? 4 : 2) * STAGE];
   __shared__ uint32_t lst[kF32MaxTiles];
 
   const int vid = xcd_remap(blockIdx.x, p.B * p.H, p.nqt);
@@ -905,7 +965,8 @@ __global__ __launch_bounds__(256, 1) void dq32_kernel(const Params p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5, c32 = lane & 31;
   const int q0 = qt * BM;
-  const int qw0 = q0 + wave * 32;
+  const int cw = SPLIT ? 0 : wave;  // wave of those that share a tile
+  const int qw0 = q0 + cw * 32;
   const int qrow = qw0 + c32;
   const bool qok = qrow < p.Lq;
   const int qc = qok ? qrow : p.Lq - 1;
@@ -940,8 +1001,8 @@ __global__ __launch_bounds__(256, 1) void dq32_kernel(const Params p) {
     for (int r = 0; r < 16; ++r) dq[db][r] = 0.f;
 
   S ks, vs_;
-  ks.init(p.k_str[2], p.D, wave, lane);
-  vs_.init(p.v_str[2], p.Dv, wave, lane);
+  ks.init(p.k_str[2], p.D, cw, lane);
+  vs_.init(p.v_str[2], p.Dv, cw, lane);
   F32Offsets<DP> lo;
   lo.init(g, c32);
   const uint32_t lds0 = lds_offset(smem);
@@ -952,23 +1013,31 @@ __global__ __launch_bounds__(256, 1) void dq32_kernel(const Params p) {
     const i32x4 rv = tile_rsrc<BN>(vp, p.v_str[2], t * BN, p.Lk, p.Dv);
 #pragma unroll
     for (int m = 0; m < S::CNT; ++m) {
-      ks.issue(rk, at, m, wave);
-      vs_.issue(rv, at + TILE, m, wave);
+      ks.issue(rk, at, m, cw);
+      vs_.issue(rv, at + TILE, m, cw);
     }
   };
 
   const int64_t brow = p.has_bias ? b * p.bias_str[0] + h * p.bias_str[1] + (int64_t)qc * p.bias_str[2] : 0;
   const uint8_t* mrow = p.has_mask ? p.mask + b * p.mask_str[0] + h * p.mask_str[1] + (int64_t)qc * p.mask_str[2] : nullptr;
 
-  if (n > 0) issue(0, 0);
-  __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-  __syncthreads();
-  for (int i = 0; i < n; ++i) {
-    const int st = i & 1;
+  if constexpr (!SPLIT) {
+    if (n > 0) issue(0, 0);
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    __syncthreads();
+  }
+  for (int i = SPLIT ? wave : 0; i < n; i += SPLIT ? 4 : 1) {
+    const int st = SPLIT ? wave : i & 1;
     const uint32_t at = lds0 + st * STAGE;
     const int t = (int)(lst[i] & 0xffff), cls = (int)(lst[i] >> 16);
     const int k0 = t * BN;
-    issue(i + 1, st ^ 1);
+    if constexpr (SPLIT) {
+      // Only this wave reads its stage: its own wait publishes the copies.
+      issue(i, st);
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    } else {
+      issue(i + 1, st ^ 1);
+    }
 
     constexpr int NA = 2 * NKB;  // S^T of each 32-key block, then dP^T
     f32x16 acc[NA];
@@ -1063,8 +1132,41 @@ __global__ __launch_bounds__(256, 1) void dq32_kernel(const Params p) {
       __builtin_amdgcn_sched_group_barrier(kSchedMfma, 8 * NDH, 0);
     }
 
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    if constexpr (SPLIT) {
+      // The next copies overwrite the stage the products just read.
+      __builtin_amdgcn_s_waitcnt(lgkmcnt_imm(0));
+    } else {
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+      __syncthreads();
+    }
+  }
+
+  if constexpr (SPLIT) {
+    // Sums of the four waves, [field][wave][lane] floats, into waves 0, 1's
+    // column block.
     __syncthreads();
+    float* ms = reinterpret_cast<float*>(smem);
+    static_assert(NDB * 16 * 4 * 64 * 4 <= 4 * STAGE && NDB == 2, "the sums fit the stages");
+    auto slot = [&](int f, int w) -> float& { return ms[(f * 4 + w) * 64 + lane]; };
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) slot(db * 16 + r, wave) = dq[db][r];
+    __syncthreads();
+    if (wave >= NDB || !qok) return;
+    f32x16 o;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int f = wave * 16 + r;
+      o[r] = (slot(f, 0) + slot(f, 1)) + (slot(f, 2) + slot(f, 3));
+    }
+    float* dqp = (float*)p.dq + b * p.q_str[0] + h * p.q_str[1] + (int64_t)qrow * p.q_str[2];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int d0 = wave * 32 + 8 * c + 4 * g;
+      if (d0 < p.D) store4(dqp + d0, o, 4 * c, p.scale);
+    }
+    return;
   }
 
   if (qok) {
@@ -1131,10 +1233,31 @@ bool launch_fwd32(Params p, int dp, hipStream_t stream) {
   return true;
 }
 
+// Whether a backward launch of `blocks` 128-row blocks that stream n rows
+// takes the split variant: with at most 128 blocks half the CUs are idle and
+// every wave walks a serial chain of tiles at one wave per SIMD.  Split, a
+// block has 32 stationary rows and each wave every fourth 32-row tile: four
+// times the blocks, two on a CU (67 KB of LDS, 256 registers), at a quarter of
+// the chain.  Head dim 64, us of dK/dV and dQ: 72 blocks, 344 rows 83 + 57 ->
+// 42 + 31; 32 blocks, 1024 rows 197 + 137 -> 65 + 42; 128 blocks, 128 rows
+// 34 + 26 -> 22 + 17, 2048 rows 390 + 267 -> 170 + 123.
+static bool split32(int64_t blocks, int n) {
+  return blocks <= 128 && n > 64 && (n + 31) / 32 <= kF32MaxTiles;
+}
+
 bool launch_dkdv32(Params p, int dp, hipStream_t stream) {
   const int bq = dp > 128 ? 32 : 64;
   if (dp > 256 || (p.Lq + bq - 1) / bq > kF32MaxTiles) return false;
   p.nkt = (p.Lk + 127) / 128;
+  if (dp == 64 && split32(p.nbh * p.nkt, p.Lq)) {
+    p.nkt = (p.Lk + 31) / 32;
+    const dim3 grid(p.nbh * p.nkt);
+    if (p.causal)
+      hipLaunchKernelGGL((dkdv32_kernel<64, true, kF32Both, true>), grid, dim3(256), 0, stream, p);
+    else
+      hipLaunchKernelGGL((dkdv32_kernel<64, false, kF32Both, true>), grid, dim3(256), 0, stream, p);
+    return true;
+  }
   const dim3 grid(p.nbh * p.nkt);
   if (dp == 256) {
     // dV, then dK and dbias.
@@ -1159,6 +1282,13 @@ bool launch_dq32(Params p, int dp, hipStream_t stream) {
   const int bn = dp > 128 ? 32 : 64;
   if (dp > 256 || (p.Lk + bn - 1) / bn > kF32MaxTiles) return false;
   p.nqt = (p.Lq + 127) / 128;
+  if (dp == 64 && split32(p.B * p.H * p.nqt, p.Lk)) {
+    p.nqt = (p.Lq + 31) / 32;
+    const dim3 grid(p.B * p.H * p.nqt);
+    if (p.causal) hipLaunchKernelGGL((dq32_kernel<64, true, true>), grid, dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL((dq32_kernel<64, false, true>), grid, dim3(256), 0, stream, p);
+    return true;
+  }
   const dim3 grid(p.B * p.H * p.nqt);
   if (dp == 64) {
     if (p.causal) hipLaunchKernelGGL((dq32_kernel<64, true>), grid, dim3(256), 0, stream, p);
