@@ -40,6 +40,8 @@
 #include "nxa_fwd16.h"
 #include "nxa_launch.h"
 
+#include <type_traits>
+
 namespace nxa {
 
 namespace {
@@ -172,13 +174,44 @@ __device__ __forceinline__ void mask_block(f32x16& x, uint32_t w, int key0, int 
   }
 }
 
+// Logits beyond this magnitude (log2 units) step by more than one unit in
+// fp32: a product of which only one side is rounded (the exponent's FMA
+// against a rounded reference) would be off by whole powers of two there, up
+// to 2^64 at a bias of -1e9.  Both sides are then rounded alike.
+constexpr float kBigLogit = 16777216.f;
+
+// x cc + r with x cc rounded first (no contraction).
+__device__ __forceinline__ float rounded_fma(float x, float cc, float r) {
+#pragma clang fp contract(off)
+  const float y = x * cc;
+  return y + r;
+}
+
+// Exponents of a block's P from its scores x and -lse log2(e) of row r in
+// nl(r).  BIG (some row's lse is beyond kBigLogit: masked throughout by a
+// large finite bias): x cc is rounded as the reference was, and the exponent
+// is held at 0, as no P is larger than 1 (a NaN stays one).
+template <bool BIG, typename NL>
+__device__ __forceinline__ void p_exponents(f32x16& x, float cc, NL&& nl) {
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    if constexpr (BIG) {
+      const float e = rounded_fma(x[r], cc, nl(r));
+      x[r] = e > 0.f ? 0.f : e;
+    } else {
+      x[r] = __builtin_fmaf(x[r], cc, nl(r));
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Packs bias / scale (fp32) into accumulator blocks.  One block of threads
 // per 32 x 32 block; blockIdx.y 0 writes the S^T layout (lane = query, rows
 // = keys; keys past Lk are -inf, which masks the tail), 1 the S layout
-// (lane = key, rows = queries).  A finite bias whose quotient would overflow
-// keeps the largest finite magnitude, so that rows masked throughout with
-// the type's lowest value stay rows of equal finite logits.
+// (lane = key, rows = queries).  Finite biases whose quotient would overflow
+// (or leave no room for the products) are mapped, in order and apart, onto
+// [2^127, 2^128): a row masked throughout with the type's lowest value stays
+// a row of equal finite logits, and a larger one in it still wins.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void bias_pack_kernel(const Params p, const ShortParams s) {
   const int lane = threadIdx.x & 63, c = threadIdx.x >> 6;
@@ -198,7 +231,9 @@ __global__ __launch_bounds__(256) void bias_pack_kernel(const Params p, const Sh
                                  ob * p.bias_str[0] + oh * p.bias_str[1] +
                                      (int64_t)q * p.bias_str[2] + key);
       x = bv * s.inv_scale;
-      if (__builtin_isfinite(bv)) x = fminf(fmaxf(x, -3.402823466e38f), 3.402823466e38f);
+      const float half = 1.70141183e38f;  // 2^127
+      if (__builtin_isfinite(bv) && !(fabsf(x) <= half))
+        x = __builtin_copysignf(__builtin_fmaf(0.499f, fabsf(bv), half), bv);
     }
     v[j] = x;
   }
@@ -252,6 +287,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_short_kernel(const Params p, c
 #pragma unroll
     for (int db = 0; db < NDB; ++db) oacc[db] = splat16(0.f);
     float m_ref = -INFINITY, l_i = 0.f;
+    bool big = false;  // a biased row's reference is beyond kBigLogit
     const int64_t blk0 = HAS_BIAS ? ((int64_t)bias_slot(sp, b, h) * sp.nqb + st) * sp.nkb : 0;
     const int nk = CAUSAL ? min(nkt, (q0 + 31) / 64 + 1) : nkt;
     for (int kt = 0; kt < nk; ++kt) {
@@ -284,7 +320,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_short_kernel(const Params p, c
       // in force and redone with a raised one only when a half-row sum
       // leaves the fp16 range of P (or the row has no reference yet).
       Frag pf[2][FPB];
-      auto exp_tile = [&]() NXA_INLINE -> float {
+      auto exp_tile = [&](auto big_tag) NXA_INLINE -> float {
         const float neg_m = m_ref == -INFINITY ? 0.f : -m_ref;
         float ts = 0.f;
 #pragma unroll
@@ -293,7 +329,8 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_short_kernel(const Params p, c
           float rs[4];
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            pt[r] = fast_exp2(__builtin_fmaf(S[kb][r], cc, neg_m));
+            pt[r] = fast_exp2(decltype(big_tag)::value ? rounded_fma(S[kb][r], cc, neg_m)
+                                                       : __builtin_fmaf(S[kb][r], cc, neg_m));
             rs[r & 3] = r < 4 ? pt[r] : rs[r & 3] + pt[r];
           }
           ts += (rs[0] + rs[1]) + (rs[2] + rs[3]);
@@ -303,9 +340,9 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_short_kernel(const Params p, c
         return ts;
       };
       float ts = 0.f;
-      bool redo = __any(m_ref == -INFINITY);
+      bool redo = big || __any(m_ref == -INFINITY);
       if (!redo) {
-        ts = exp_tile();
+        ts = exp_tile(std::false_type{});
         redo = __any(!(ts <= kFwdSumLimit));
       }
       if (redo) {
@@ -325,7 +362,8 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_short_kernel(const Params p, c
 #pragma unroll
             for (int r = 0; r < 16; ++r) oacc[db][r] *= alpha;
         }
-        ts = exp_tile();
+        big = HAS_BIAS && __any(m_ref != -INFINITY && fabsf(m_ref) > kBigLogit);
+        ts = big ? exp_tile(std::true_type{}) : exp_tile(std::false_type{});
       }
       l_i += ts;
       const uint32_t vat = v_lds + kt * TILE_BYTES;
@@ -410,6 +448,7 @@ __global__ __launch_bounds__(NW * 64, 2) void dq_short_kernel(const Params p, co
     const int64_t rowid = ((int64_t)b * p.H + h) * p.Lq + qc;
     const float ndlt = -(dacc + shfl_xor32(dacc));
     const float nlse2 = -p.lse[rowid] * kLog2e;
+    const bool big = HAS_BIAS && __any(fabsf(nlse2) > kBigLogit);
     if (qok && g == 0) {
       p.ndelta[rowid] = ndlt;
       p.nlse2[rowid] = nlse2;
@@ -422,40 +461,44 @@ __global__ __launch_bounds__(NW * 64, 2) void dq_short_kernel(const Params p, co
     for (int db = 0; db < NDB; ++db) dq[db] = splat16(0.f);
     const int64_t blk0 = HAS_BIAS ? ((int64_t)bias_slot(sp, b, h) * sp.nqb + st) * sp.nkb : 0;
     const int nk = CAUSAL ? min(nkt, (q0 + 31) / 64 + 1) : nkt;
-    for (int kt = 0; kt < nk; ++kt) {
-      const KeepBits kb2 = {(uint32_t)__builtin_amdgcn_readfirstlane((int)kbits[2 * kt]),
-                            (uint32_t)__builtin_amdgcn_readfirstlane((int)kbits[2 * kt + 1])};
-      if (!kb2.any()) continue;
-      const int k0 = kt * 64;
-      const bool diag = CAUSAL && k0 + 63 > q0;
-      const bool masked = diag || (!kb2.all() && (!HAS_BIAS || p.has_mask));
+    const auto tiles = [&](auto big_tag) NXA_INLINE {
+      for (int kt = 0; kt < nk; ++kt) {
+        const KeepBits kb2 = {(uint32_t)__builtin_amdgcn_readfirstlane((int)kbits[2 * kt]),
+                              (uint32_t)__builtin_amdgcn_readfirstlane((int)kbits[2 * kt + 1])};
+        if (!kb2.any()) continue;
+        const int k0 = kt * 64;
+        const bool diag = CAUSAL && k0 + 63 > q0;
+        const bool masked = diag || (!kb2.all() && (!HAS_BIAS || p.has_mask));
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        const uint32_t kat = k_lds + kt * TILE_BYTES + kb * HALF;
-        const uint32_t vat = v_lds + kt * TILE_BYTES + kb * HALF;
-        f32x16 s, dp = nd16;
-        if constexpr (HAS_BIAS) s = packed_block(sp.pack_st, blk0 + 2 * kt + kb, lane);
+        for (int kb = 0; kb < 2; ++kb) {
+          const uint32_t kat = k_lds + kt * TILE_BYTES + kb * HALF;
+          const uint32_t vat = v_lds + kt * TILE_BYTES + kb * HALF;
+          f32x16 s, dp = nd16;
+          if constexpr (HAS_BIAS) s = packed_block(sp.pack_st, blk0 + 2 * kt + kb, lane);
 #pragma unroll
-        for (int m = 0; m < NC; ++m) {
-          const Frag a = rd.row(kat, m);
-          if (!HAS_BIAS && m == 0) s = M::first(a, qf[m]);
-          else M::run(s, a, qf[m]);
-          M::run(dp, rd.row(vat, m), df[m]);
-        }
+          for (int m = 0; m < NC; ++m) {
+            const Frag a = rd.row(kat, m);
+            if (!HAS_BIAS && m == 0) s = M::first(a, qf[m]);
+            else M::run(s, a, qf[m]);
+            M::run(dp, rd.row(vat, m), df[m]);
+          }
+          const auto row_nl = [&](int) NXA_INLINE { return nlse2; };
+          p_exponents<decltype(big_tag)::value>(s, p.scale_log2, row_nl);
+          if (masked)
+            mask_block<CAUSAL>(s, (kb ? kb2.hi : kb2.lo) >> (4 * g), k0 + 32 * kb + 4 * g, qrow);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] = __builtin_fmaf(s[r], p.scale_log2, nlse2);
-        if (masked)
-          mask_block<CAUSAL>(s, (kb ? kb2.hi : kb2.lo) >> (4 * g), k0 + 32 * kb + 4 * g, qrow);
+          for (int r = 0; r < 16; ++r) dp[r] = fast_exp2(s[r]) * dp[r];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) dp[r] = fast_exp2(s[r]) * dp[r];
+          for (int f = 0; f < FPB; ++f) {
+            const Frag pd = M::pack(dp, f);
 #pragma unroll
-        for (int f = 0; f < FPB; ++f) {
-          const Frag pd = M::pack(dp, f);
-#pragma unroll
-          for (int db = 0; db < NDB; ++db) M::run(dq[db], rd.tr(kat, f, db), pd);
+            for (int db = 0; db < NDB; ++db) M::run(dq[db], rd.tr(kat, f, db), pd);
+          }
         }
       }
-    }
+    };
+    if (big) tiles(std::true_type{});
+    else tiles(std::false_type{});
     if (qok) {
       T* dqp = (T*)p.dq + b * p.q_str[0] + h * p.q_str[1] + (int64_t)qrow * p.q_str[2];
 #pragma unroll
@@ -474,7 +517,7 @@ __global__ __launch_bounds__(NW * 64, 2) void dq_short_kernel(const Params p, co
 // 32-key strips.  Rows past Lq read as zeros with -lse2 = -inf, so P = 0.
 // ---------------------------------------------------------------------------
 template <typename T, int DP, int NW, bool HAS_BIAS, bool CAUSAL>
-__global__ __launch_bounds__(NW * 64, 2) void dkdv_short_kernel(const Params p, const ShortParams sp) {
+__global__ __launch_bounds__(NW * 64, DP == 32 && !CAUSAL ? 4 : 2) void dkdv_short_kernel(const Params p, const ShortParams sp) {
   using M = Mma<T>;
   using Frag = typename M::Frag;
   constexpr int NC = DP / 16, NDB = DP / 32, FPB = M::FRAGS_PER_BLOCK;
@@ -496,14 +539,18 @@ __global__ __launch_bounds__(NW * 64, 2) void dkdv_short_kernel(const Params p, 
   load_resident<DP, NW>((const T*)p.dout + b * p.o_str[0] + h * p.o_str[1], p.o_str[2], p.Lq, nqt, p.Dv,
                     d_lds, wave, lane);
   const int64_t row0 = ((int64_t)b * p.H + h) * p.Lq;
+  bool far = false;  // a row's lse beyond kBigLogit
   for (int i = tid; i < nqt * 64; i += NW * 64) {
     nl_s[i] = i < p.Lq ? p.nlse2[row0 + i] : -INFINITY;
     nd_s[i] = i < p.Lq ? p.ndelta[row0 + i] : 0.f;
+    if (HAS_BIAS) far = far || (i < p.Lq && fabsf(nl_s[i]) > kBigLogit);
   }
   Resident<T, DP> rd;
   rd.init(lane);
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-  __syncthreads();
+  bool big = false;
+  if constexpr (HAS_BIAS) big = __syncthreads_or(far);
+  else __syncthreads();
 
   const int nqb = (p.Lq + 31) / 32;
   for (int st = part * NW + wave; st < nst; st += sp.nsplit * NW) {
@@ -522,53 +569,60 @@ __global__ __launch_bounds__(NW * 64, 2) void dkdv_short_kernel(const Params p, 
     for (int db = 0; db < NDB; ++db) dk[db] = dv[db] = splat16(0.f);
     const int64_t slot0 = HAS_BIAS ? (int64_t)bias_slot(sp, b, h) * sp.nqb : 0;
     const bool some = __any(keep), every = __all(keep);
-    for (int qb = CAUSAL ? st : 0; qb < (some ? nqb : 0); ++qb) {
-      const uint32_t qat = q_lds + qb * HALF, dat = d_lds + qb * HALF;
-      f32x16 x, d;
-      float nl[16];
+    const auto blocks = [&](auto big_tag) NXA_INLINE {
+      for (int qb = CAUSAL ? st : 0; qb < (some ? nqb : 0); ++qb) {
+        const uint32_t qat = q_lds + qb * HALF, dat = d_lds + qb * HALF;
+        f32x16 x, d;
+        float nl[16];
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const f32x4 l4 = *reinterpret_cast<const f32x4*>(nl_s + qb * 32 + 8 * c + 4 * g);
-        const f32x4 d4 = *reinterpret_cast<const f32x4*>(nd_s + qb * 32 + 8 * c + 4 * g);
+        for (int c = 0; c < 4; ++c) {
+          const f32x4 l4 = *reinterpret_cast<const f32x4*>(nl_s + qb * 32 + 8 * c + 4 * g);
+          const f32x4 d4 = *reinterpret_cast<const f32x4*>(nd_s + qb * 32 + 8 * c + 4 * g);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          nl[4 * c + j] = l4[j];
-          d[4 * c + j] = d4[j];
+          for (int j = 0; j < 4; ++j) {
+            nl[4 * c + j] = l4[j];
+            d[4 * c + j] = d4[j];
+          }
         }
-      }
-      if constexpr (HAS_BIAS) x = packed_block(sp.pack_s, (slot0 + qb) * sp.nkb + st, lane);
+        if constexpr (HAS_BIAS) x = packed_block(sp.pack_s, (slot0 + qb) * sp.nkb + st, lane);
 #pragma unroll
-      for (int m = 0; m < NC; ++m) {
-        const Frag a = rd.row(qat, m);
-        if (!HAS_BIAS && m == 0) x = M::first(a, kf[m]);
-        else M::run(x, a, kf[m]);
-        M::run(d, rd.row(dat, m), vf[m]);
-      }
+        for (int m = 0; m < NC; ++m) {
+          const Frag a = rd.row(qat, m);
+          if (!HAS_BIAS && m == 0) x = M::first(a, kf[m]);
+          else M::run(x, a, kf[m]);
+          M::run(d, rd.row(dat, m), vf[m]);
+        }
+        // (read late in the rare variant: registers)
+        const auto row_nl = [&](int r) NXA_INLINE {
+          return decltype(big_tag)::value ? nl_s[qb * 32 + 8 * (r >> 2) + 4 * g + (r & 3)] : nl[r];
+        };
+        p_exponents<decltype(big_tag)::value>(x, p.scale_log2, row_nl);
+        if (!every || (CAUSAL && qb == st)) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) x[r] = __builtin_fmaf(x[r], p.scale_log2, nl[r]);
-      if (!every || (CAUSAL && qb == st)) {
+          for (int r = 0; r < 16; ++r) {
+            bool kp = keep;
+            if (CAUSAL) kp = kp && key <= qb * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
+            x[r] = kp ? x[r] : -INFINITY;
+          }
+        }
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          bool kp = keep;
-          if (CAUSAL) kp = kp && key <= qb * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
-          x[r] = kp ? x[r] : -INFINITY;
+          x[r] = fast_exp2(x[r]);
+          d[r] = x[r] * d[r];
+        }
+#pragma unroll
+        for (int f = 0; f < FPB; ++f) {
+          const Frag pp = M::pack(x, f), pd = M::pack(d, f);
+#pragma unroll
+          for (int db = 0; db < NDB; ++db) {
+            M::run(dv[db], rd.tr(dat, f, db), pp);
+            M::run(dk[db], rd.tr(qat, f, db), pd);
+          }
         }
       }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        x[r] = fast_exp2(x[r]);
-        d[r] = x[r] * d[r];
-      }
-#pragma unroll
-      for (int f = 0; f < FPB; ++f) {
-        const Frag pp = M::pack(x, f), pd = M::pack(d, f);
-#pragma unroll
-        for (int db = 0; db < NDB; ++db) {
-          M::run(dv[db], rd.tr(dat, f, db), pp);
-          M::run(dk[db], rd.tr(qat, f, db), pd);
-        }
-      }
-    }
+    };
+    if (big) blocks(std::true_type{});
+    else blocks(std::false_type{});
     if (kok) {
       T* dkp = (T*)p.dk + b * p.k_str[0] + h * p.k_str[1] + (int64_t)key * p.k_str[2];
       T* dvp = (T*)p.dv + b * p.v_str[0] + h * p.v_str[1] + (int64_t)key * p.v_str[2];
@@ -719,8 +773,9 @@ __global__ __launch_bounds__(kDbiasWaves<DP> * 64, DP == 32 ? 3 : 2) void dbias_
         M::run(s, rd.row(kat, m), rd.row(qat + qb * HALF, m));
         M::run(dp, rd.row(kat + KMAT, m), rd.row(qat + MAT + qb * HALF, m));
       }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = __builtin_fmaf(s[r], p.scale_log2, nlse2);
+      const auto row_nl = [&](int) NXA_INLINE { return nlse2; };
+      if (__any(fabsf(nlse2) > kBigLogit)) p_exponents<true>(s, p.scale_log2, row_nl);
+      else p_exponents<false>(s, p.scale_log2, row_nl);
       if (diag || keep != 0xffffffffu)
         mask_block<CAUSAL>(s, keep >> (4 * g), k0 + 4 * g, q0 + 32 * qb + c32);
 #pragma unroll

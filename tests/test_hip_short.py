@@ -11,7 +11,8 @@ from __future__ import annotations
 import numpy as np
 import pytest
 import torch
-from test_hip_parity import _check, _dev, _draw, _to
+from _golden import relerr
+from test_hip_parity import REL, _check, _dev, _draw, _to
 
 pytestmark = pytest.mark.gpu
 
@@ -65,6 +66,54 @@ def test_large_and_negative_infinite_bias(dtype):
     got = out.float().cpu().numpy()
     assert np.isfinite(got).all()
     assert np.abs(got - ref).max() / np.abs(ref).max() <= (2e-2 if dtype == BF else 2e-3)
+
+
+LOWEST = float(np.finfo(np.float32).min)
+
+
+@pytest.mark.parametrize('dtype, bias_dtype', [(HF, F32), (BF, F32), (BF, BF)],
+                         ids=['f16', 'bf16', 'bf16b'])
+@pytest.mark.parametrize('d', [16, 24, 32, 40, 64])
+@pytest.mark.parametrize('const', [-1e4, -1e9, -1e10, -1e30, LOWEST])
+def test_large_finite_bias_as_a_mask(dtype, bias_dtype, d, const):
+    """A shared bias that masks with a large finite constant: on the first
+    keys (the first tiles hold nothing else), on the last, and on whole rows.
+    The whole rows' output is the softmax of what float32 keeps of their
+    scores (from 1e8 on nothing: the mean of v), and with a zero cotangent
+    they leave every gradient alone."""
+    from nitrix_amd import scaled_dot_product_attention
+    from oracle import attention as O
+
+    rng = np.random.default_rng(d)
+    B, H, s, t = 72, 4, 40, 131
+    q, k, v, g = (_draw(rng, (B, H, n, d), dtype) for n in (s, t, t, s))
+    bias = _draw(rng, (1, H, s, t), bias_dtype)
+    if bias_dtype == BF:
+        const = max(const, float(torch.finfo(BF).min))
+        const = float(torch.tensor(const).to(BF))
+    bias[:, :, :20, :64] = const
+    bias[:, :, 20:30] = const
+    bias[:, :, 30:, 70:] = const
+    if const < -1e38:
+        bias[:, :, 29, 100:] = const / 2  # larger: these keys take the row
+    g[:, :, 20:30] = 0
+    tq, tk, tv, tb = _to(q, dtype, True), _to(k, dtype, True), _to(v, dtype, True), _to(bias, bias_dtype, True)
+    print(f'[case] {dtype} {bias_dtype} d{d} const {const}', flush=True)
+    out = scaled_dot_product_attention(tq, tk, tv, bias=tb, backend='hip')
+    grads = torch.autograd.grad(out, (tq, tk, tv, tb), _to(g, dtype))
+    b64 = np.broadcast_to(bias, (B, H, s, t)).astype(np.float64)
+    ref = O.sdpa_forward(q, k, v, bias=b64, scale=d ** -0.5, acc_dtype=np.float64)
+    if const < -1e8:
+        ref[:, :, 20:30] = v.astype(np.float64).mean(2, keepdims=True)
+    if const < -1e38:
+        ref[:, :, 29] = v[:, :, 100:].astype(np.float64).mean(2)
+    want = O.sdpa_backward(q, k, v, g, bias=bias, scale=d ** -0.5, acc_dtype=np.float64)
+    for name, got, w in zip(('out', 'dq', 'dk', 'dv', 'dbias'), (out, *grads), (ref, *want)):
+        got = got.detach().float().cpu().numpy()
+        assert np.isfinite(got).all(), name
+        err = relerr(got, w.reshape(got.shape))
+        tol = max(REL[dtype], REL[bias_dtype]) if name == 'dbias' else REL[dtype]
+        assert err <= tol, (name, err)
 
 
 def test_workspace_without_room_for_the_packed_bias():
