@@ -216,9 +216,10 @@ __global__ __launch_bounds__(256, 2) void fwd_split_kernel(const Params p, const
 #pragma unroll
     for (int r = 1; r < 16; ++r) mt = fmaxf(mt, s[r]);
     mt = fmaxf(mt, shfl_xor32(mt));
-    const float mn = fmaxf(m_ref, mt);  // finite or +inf: a listed tile keeps a key
+    const float mn = fmaxf(m_ref, mt);
     if (__any(mn > m_ref)) {
-      const float alpha = fast_exp2(m_ref - mn);
+      // (a row whose kept scores are all -inf so far keeps -inf: no factor)
+      const float alpha = mn > m_ref ? fast_exp2(m_ref - mn) : 1.f;
       l_i *= alpha;
 #pragma unroll
       for (int db = 0; db < NDB; ++db)

@@ -52,3 +52,32 @@ def test_masks_that_empty_splits_and_batches():
                          acc_dtype=np.float64)
     assert np.isfinite(got[keep]).all()
     assert np.abs(got[keep] - ref).max() / np.abs(ref).max() <= 2e-2
+
+
+@pytest.mark.parametrize('dtype', [BF, HF], ids=['bf16', 'f16'])
+@pytest.mark.parametrize('t', [545, 9000])
+def test_scores_of_minus_infinity(dtype, t):
+    """A wave whose only kept key scores -inf for half of the rows (an
+    overflowing bf16 product, an infinite fp16 key) and more for the others:
+    the key weighs nothing in those rows."""
+    rng = np.random.default_rng(7)
+    B, H, s, d = 2, 2, 20, 64
+    q, k, v = (_draw(rng, (B, H, n, d), dtype) for n in (s, t, t))
+    lone = t - 1 if t == 545 else 40
+    mask = np.zeros((1, 1, 1, t), bool)
+    mask[..., :20] = mask[..., lone] = True
+    k[..., lone, :] = 0
+    k[..., lone, 5] = 3e38 if dtype == BF else np.inf
+    q[..., ::2, 5] = -2
+    q[..., 1::2, 5] = 0 if dtype == BF else 1
+    k[..., :20, 5] = 0
+    rows = slice(None) if dtype == BF else slice(0, None, 2)
+    from nitrix_amd import scaled_dot_product_attention
+    from oracle import attention as O
+
+    out = scaled_dot_product_attention(_to(q, dtype), _to(k, dtype), _to(v, dtype),
+                                       mask=torch.from_numpy(mask).to(_dev()), backend='hip')
+    got = out.float().cpu().numpy()[:, :, rows]
+    ref = O.sdpa_forward(q[:, :, rows], k, v, mask=mask, scale=d ** -0.5, acc_dtype=np.float64)
+    assert np.isfinite(got).all()
+    assert np.abs(got - ref).max() / np.abs(ref).max() <= (2e-2 if dtype == BF else 2e-3)
