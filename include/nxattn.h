@@ -111,7 +111,8 @@ int nxa_check(const nxa_desc* desc, int has_bias, int has_mask);
  * and keys and head dims of at most 64 whose bias is shared by at least four
  * (batch, head) pairs (and whose mask, if any, broadcasts over queries),
  * room for the bias packed in fp32 (padded to whole 64 x 64 tiles; twice in
- * the backward), and for a forward of at most 64 queries over more than 512
+ * the backward) where packing it is faster (a rule on the descriptor: pairs,
+ * pairs that share, lengths, dtypes and strides), and for a forward of at most 64 queries over more than 512
  * keys (bf16 / fp16, head dims of at most 128, no bias, not causal, the same
  * masks) room for the partial results of its key splits (fp32, one padded
  * output per 32 queries and split); without that room such a problem is

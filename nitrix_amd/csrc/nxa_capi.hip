@@ -228,18 +228,70 @@ DbiasGeom dbias_geom(const nxa_desc* d) {
   return g;
 }
 
+int fwd_bias_mode(const nxa_desc* d, const void* bias, float* h, float* l);
+bool bias_rows_vec(const nxa_desc* d, const void* bias);
+
 // Short-sequence path (nxa_short16.hip): 16-bit I/O, both head dims at most
 // 64, at most kShortMax queries and keys, a mask (if any) that broadcasts
 // over queries, and a bias (if any) shared by at least four (batch, head)
-// pairs, so that packing it costs less than the pairs' reads of it, with a
-// positive scale whose reciprocal is far from the ends of fp32's range.
-// Decided on the descriptor alone, so that a call's forward, backward and
-// workspace sizes agree.
+// pairs with a positive scale whose reciprocal is far from the ends of
+// fp32's range.  Decided on the descriptor alone, so that a call's forward,
+// backward and workspace sizes agree.  A biased problem packs its bias first
+// (fwd_pack, bwd_pack): else the general kernels take it.
 struct ShortGeom {
   bool ok;
+  bool fwd_pack, bwd_pack;
   int OB, OH, nqb, nkb;
   size_t pack_bytes;  // one layout of the packed bias
 };
+
+// Whether the forward's gain pays for the pack: a launch and 8 bytes per
+// bias element and slot, against the general forward, which reads the bias
+// in place.  Times in us (bf16 I/O, general -> packed), slots = pairs / P:
+//  * A bias that the general kernel adds on the matrix cores costs it little.
+//    Up to 256 pairs the pack is never paid for; beyond, the gain is the
+//    padding to 256-row blocks (512 pairs of 400^2, d 32, P 32: 0.65 of the
+//    general time, P 4: 1.29; 1024 pairs of 64^2, P 4: 0.75; 512 pairs of
+//    64^2, P 32: 0.94, but a call of 29 us is one of 34 on the host) and, at
+//    head dim 32, half the products (512 pairs of 512^2: P 32 0.81, P 16
+//    1.03, P 8 1.65; head dim 64: P 128 0.97, P 32 1.09, P 4 2.27).  A bias
+//    that broadcasts over queries is cheaper still (1024 pairs of 256^2,
+//    head dim 64: 1.08).
+//  * One it adds element by element gains more: 512 pairs of 343^2, P 4,
+//    309 -> 89, fp32 bias 194 -> 94; 196^2, P 32: 51 -> 27.  Small calls are
+//    bound by their launches (256 pairs of 144^2, P 4, fp32: 20 -> 26; 64
+//    pairs of 196^2: 23 -> 20, but the call 31 -> 35 on the host), and a bias
+//    of few pairs a slot that it loads four elements at a time by the pack
+//    (512^2, P 4: 155 -> 185, P 8: 155 -> 126).
+bool fwd_pays_pack(const nxa_desc* d, int64_t slots) {
+  const int64_t pairs = (int64_t)d->B * d->H, P = pairs / slots;
+  const int64_t area = (int64_t)d->Lq * d->Lk;
+  const bool short128 = d->Lq <= 128 && d->Lk <= 128;
+  float h, l;
+  // (both as for an aligned pointer)
+  if (fwd_bias_mode(d, nullptr, &h, &l) != nxa::kFbValu) {
+    if (pairs <= 256) return false;
+    const bool d32 = d->D <= 32 && value_dim(d) <= 32;
+    const bool padded = (d->Lq + 255) / 256 * 256 * 5 >= d->Lq * 6;
+    if (d->bias_str[2] == 0 && d->Lq > 1) return pairs >= 1024 && (padded || d32);
+    if (short128) return pairs >= 1024;
+    if (padded || d32) return P >= (pairs >= 1024 ? 16 : 32);
+    return P >= 64;
+  }
+  const bool small = (pairs <= 256 && area <= 256 * 256) || (pairs < 1024 && area <= 64 * 64);
+  if (!bias_rows_vec(d, nullptr)) return !small || esize(d->bias_dtype) == 2;
+  if (small) return false;
+  return pairs <= 64 || P >= 8 || area <= 200 * 200;
+}
+
+// The backward packs twice and still gains with every bias but one that
+// broadcasts over queries at few pairs (dK / dV then form no dbias here):
+// 64 pairs of 512^2, frozen bias, 1.39 of the general time, of 64^2 1.2.
+bool bwd_pays_pack(const nxa_desc* d) {
+  if (d->bias_str[2] != 0 || d->Lq == 1 || (int64_t)d->B * d->H > 256) return true;
+  float h, l;
+  return fwd_bias_mode(d, nullptr, &h, &l) == nxa::kFbValu && (d->Lq > 128 || d->Lk > 128);
+}
 
 ShortGeom short_geom(const nxa_desc* d, int has_bias, int has_mask) {
   ShortGeom g{};
@@ -255,8 +307,11 @@ ShortGeom short_geom(const nxa_desc* d, int has_bias, int has_mask) {
   if (has_bias) {
     g.OB = d->bias_str[0] == 0 ? 1 : d->B;
     g.OH = d->bias_str[1] == 0 ? 1 : d->H;
-    if ((int64_t)d->B * d->H < 4 * (int64_t)g.OB * g.OH) g.ok = false;
-    g.pack_bytes = (size_t)g.OB * g.OH * g.nqb * g.nkb * 1024 * sizeof(float);
+    const int64_t slots = (int64_t)g.OB * g.OH;
+    if ((int64_t)d->B * d->H < 4 * slots) g.ok = false;
+    g.pack_bytes = (size_t)slots * g.nqb * g.nkb * 1024 * sizeof(float);
+    g.fwd_pack = g.ok && fwd_pays_pack(d, slots);
+    g.bwd_pack = g.ok && bwd_pays_pack(d);
   }
   return g;
 }
@@ -312,9 +367,11 @@ WsLayout ws_layout(const nxa_desc* d, int has_bias, int has_mask, int flags) {
   }
   if (has_bias && (flags & NXA_WS_PACK)) {
     // Packed bias: the S^T layout, and in the backward the S layout after it.
+    // (A backward's room also serves the forward, packing or not.)
     const ShortGeom g = short_geom(d, has_bias, has_mask);
     w.pack = off;
-    if (g.ok) off += (flags & NXA_WS_BWD ? 2 : 1) * align256(g.pack_bytes);
+    if (flags & NXA_WS_BWD ? g.bwd_pack || g.fwd_pack : g.fwd_pack)
+      off += (flags & NXA_WS_BWD ? 2 : 1) * align256(g.pack_bytes);
   }
   if (!has_bias && (flags & NXA_WS_PACK)) {
     // Partial results of the key-split forward (never beside a packed bias).
@@ -392,6 +449,13 @@ int fwd_bias_mode(const nxa_desc* d, const void* bias, float* h, float* l) {
   return nxa::kFbTile;
 }
 
+// Whether four bias elements load at once.
+bool bias_rows_vec(const nxa_desc* d, const void* bias) {
+  bool vec = d->Lk % 4 == 0 && aligned(bias, 4 * esize(d->bias_dtype));
+  for (int i = 0; i < 3; ++i) vec = vec && d->bias_str[i] % 4 == 0;
+  return vec;
+}
+
 nxa::Params base_params(const nxa_desc* d, const void* q, const void* k,
                         const void* v, const void* bias, const uint8_t* mask) {
   nxa::Params p;
@@ -422,12 +486,7 @@ nxa::Params base_params(const nxa_desc* d, const void* q, const void* k,
   p.causal = d->causal ? 1 : 0;
   p.has_bias = bias != nullptr;
   p.bias_dtype = d->bias_dtype;
-  if (bias) {
-    const int bes = esize(d->bias_dtype);
-    bool vec = (d->Lk % 4 == 0) && aligned(bias, 4 * bes);
-    for (int i = 0; i < 3; ++i) vec = vec && (d->bias_str[i] % 4 == 0);
-    p.bias_vec = vec;
-  }
+  if (bias) p.bias_vec = bias_rows_vec(d, bias);
   p.fwd_bias = bias ? fwd_bias_mode(d, bias, &p.bias_h, &p.bias_l) : nxa::kFbNone;
   p.has_mask = mask != nullptr;
   if (mask) {
@@ -804,12 +863,7 @@ int run_fwd(const nxa_desc* d, const void* q, const void* k, const void* v,
     p.qn_eps = fn->eps;
   }
   const ShortGeom sg = short_geom(d, bias != nullptr, mask != nullptr);
-  // A bias that the general forward adds on the matrix cores straight from
-  // its rows saves the pack, which up to 256 pairs costs more than the
-  // short kernels gain (head dim 64, 64 pairs of 512 x 512: 18.3 us general,
-  // 22.7 packed; 256 pairs: 38 and 44; 512 pairs of 400 x 400: 74 and 67).
-  const bool direct = bias && p.fwd_bias != nxa::kFbValu && (int64_t)d->B * d->H <= 256;
-  if (sg.ok && !fn && !direct && (!bias || packs)) {
+  if (sg.ok && !fn && (!bias || (sg.fwd_pack && packs))) {
     const WsLayout w = ws_layout(d, bias != nullptr, mask != nullptr, NXA_WS_PACK);
     const nxa::ShortParams sp =
         short_params(d, sg, bias ? static_cast<uint8_t*>(workspace) + w.pack : nullptr, false);
@@ -879,7 +933,7 @@ int run_bwd(const nxa_desc* d, const void* q, const void* k, const void* v,
   const int ws_flags = NXA_WS_BWD | (dbias ? NXA_WS_DBIAS : 0);
   WsLayout ws = ws_layout(d, bias != nullptr, mask != nullptr, ws_flags | NXA_WS_PACK);
   const ShortGeom sg = short_geom(d, bias != nullptr, mask != nullptr);
-  bool use_short = sg.ok && !na;
+  bool use_short = sg.ok && !na && (!bias || sg.bwd_pack);
   if (!workspace || workspace_bytes < ws.total || !use_short) {
     // No room for the packed bias (or no use for it): the general kernels.
     use_short = use_short && !bias;

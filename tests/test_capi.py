@@ -324,3 +324,35 @@ def test_fused_q_norm_forward_rejects_what_it_cannot_take(lib):
     rc = lib.nxa_fwd_normed(ctypes.byref(d), ok, ok, ok, None, None, ok, ok, ok, ok, -1.0,
                             None, 0, None)
     assert rc == _lib.NXA_E_ARG
+
+
+@pytest.mark.parametrize('B, H, shared, L, D, bias_dtype, packs', [
+    # Bias rows the general forward reads on the matrix cores: few pairs, few
+    # pairs a slot, and a bias broadcast over queries stay with it.
+    (64, 4, 'heads', 512, 64, _lib.NXA_BF16, False),
+    (512, 4, 'batch', 512, 32, _lib.NXA_BF16, False),
+    (128, 4, 'batch', 512, 64, _lib.NXA_BF16, False),
+    (64, 8, 'batch', 512, 32, _lib.NXA_BF16, False),
+    (16, 32, 'batch', 512, 64, _lib.NXA_BF16, False),
+    (64, 16, 'row', 256, 64, _lib.NXA_BF16, False),
+    (64, 16, 'heads', 512, 64, _lib.NXA_BF16, True),
+    (16, 32, 'batch', 512, 32, _lib.NXA_BF16, True),
+    (256, 4, 'batch', 64, 32, _lib.NXA_BF16, True),
+    (512, 4, 'heads', 400, 64, _lib.NXA_BF16, True),
+    # Bias rows it reads element by element.
+    (512, 4, 'heads', 343, 32, _lib.NXA_BF16, True),
+    (16, 4, 'batch', 343, 32, _lib.NXA_F32, True),
+    (64, 4, 'batch', 144, 64, _lib.NXA_F32, False),
+    (8, 8, 'heads', 196, 32, _lib.NXA_F32, False),
+    (128, 4, 'batch', 512, 64, _lib.NXA_F32, False),
+    (64, 8, 'batch', 512, 64, _lib.NXA_F32, True),
+])
+def test_room_for_a_packed_bias_only_where_packing_pays(lib, B, H, shared, L, D, bias_dtype, packs):
+    d = _desc(B, H, L, L, D)
+    d.bias_dtype = bias_dtype
+    d.bias_str[:] = {'heads': (0, L * L, L), 'batch': (L * L, 0, L), 'row': (0, L, 0)}[shared]
+    slots = {'heads': H, 'batch': B, 'row': H}[shared]
+    tiles = (2 * -(-L // 64)) ** 2
+    base = lib.nxa_workspace_bytes(ctypes.byref(d), 1, 0, _lib.NXA_WS_FWD)
+    room = lib.nxa_workspace_bytes(ctypes.byref(d), 1, 0, _lib.NXA_WS_PACK) - base
+    assert room == (slots * tiles * 4096 if packs else 0)
