@@ -415,15 +415,31 @@ class _Prepared:
         return torch.empty(nbytes, dtype=torch.uint8, device=self.device)
 
 
+def _may_pack(prep: _Prepared) -> bool:
+    """Whether a forward may want the room of ``NXA_WS_PACK``: 16-bit calls
+    with a bias over short sequences, or with few queries over many keys.  (A
+    small biased call is bound by its launches and the host: 64 pairs of 196 x
+    196 take 31 us without the pack's launch and allocation, 35 with.)"""
+    if prep.dtype == torch.float32:
+        return False
+    if prep.bias is None:
+        return prep.s <= 64 and prep.t > 512
+    small = prep.nb * prep.h <= 256 and prep.s * prep.t <= 65536
+    return prep.s <= 512 and prep.t <= 512 and not small
+
+
 def _forward(prep: _Prepared, for_bwd: bool = False, qnorm=None):
     """Run ``nxa_fwd``; returns ``(o [nb,h,s,d], lse [nb,h,s], workspace)``.
 
     With ``for_bwd`` the workspace is sized for a backward without dbias (it
     starts with the forward's tile map, then the per-row values), so such a
     backward reuses it as is; a backward that wants dbias of a shared bias
-    allocates its larger workspace itself.  With ``qnorm = (q_hat,
-    q_rstd)`` (``prep.q`` then holds the raw rows) the kernel normalises q
-    itself (``nxa_fwd_normed``) and writes q_hat and its per-row rsqrt."""
+    allocates its larger workspace itself.  A forward with room for a packed
+    bias or for key splits leaves no tile map: its workspace ends with the
+    call (the returned one is None), not with the backward.  With ``qnorm =
+    (q_hat, q_rstd)`` (``prep.q`` then holds the raw rows) the kernel
+    normalises q itself (``nxa_fwd_normed``) and writes q_hat and its
+    per-row rsqrt."""
     lib = _lib.lib()
     o = torch.empty(
         (prep.nb, prep.h, prep.s, prep.dv), dtype=prep.dtype, device=prep.device
@@ -431,9 +447,13 @@ def _forward(prep: _Prepared, for_bwd: bool = False, qnorm=None):
     lse = torch.empty(
         (prep.nb, prep.h, prep.s), dtype=torch.float32, device=prep.device
     )
-    # Room for the packed bias (nxa_fwd_normed has no use for it).
-    pack = _lib.NXA_WS_PACK if qnorm is None else 0
-    ws = prep.workspace((_lib.NXA_WS_BWD if for_bwd else _lib.NXA_WS_FWD) | pack)
+    ws, keep = None, True
+    if qnorm is None and _may_pack(prep):
+        room = prep.workspace_bytes(_lib.NXA_WS_PACK)
+        if room > prep.workspace_bytes(_lib.NXA_WS_FWD):
+            ws, keep = torch.empty(room, dtype=torch.uint8, device=prep.device), False
+    if keep:
+        ws = prep.workspace(_lib.NXA_WS_BWD if for_bwd else _lib.NXA_WS_FWD)
     args = (ctypes.byref(prep.desc), _ptr(prep.q), _ptr(prep.k), _ptr(prep.v),
             _ptr(prep.bias), _ptr(prep.mask), _ptr(o), _ptr(lse))
     tail = (_ptr(ws), 0 if ws is None else ws.numel(), prep.stream())
@@ -442,7 +462,7 @@ def _forward(prep: _Prepared, for_bwd: bool = False, qnorm=None):
     else:
         q_hat, q_rstd = qnorm
         _lib.check(lib.nxa_fwd_normed(*args, _ptr(q_hat), _ptr(q_rstd), _QK_RMS_EPS, *tail))
-    return o, lse, ws
+    return o, lse, ws if keep else None
 
 
 def _dbias_geometry(prep: _Prepared):

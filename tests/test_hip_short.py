@@ -116,6 +116,25 @@ def test_large_finite_bias_as_a_mask(dtype, bias_dtype, d, const):
         assert err <= tol, (name, err)
 
 
+def test_the_packed_bias_is_not_kept_for_the_backward():
+    """Between forward and backward a call holds its output, the row values
+    and no packed bias (which is larger than the bias itself)."""
+    from nitrix_amd import scaled_dot_product_attention
+
+    B, H, n, d = 96, 4, 343, 32
+    q, k, v = (torch.randn(B, H, n, d, device=_dev(), dtype=BF) for _ in range(3))
+    bias = torch.randn(B, 1, n, n, device=_dev(), dtype=BF)
+    for want in (False, True):
+        q.requires_grad_(True)
+        bias.requires_grad_(want)
+        before = torch.cuda.memory_allocated()
+        out = scaled_dot_product_attention(q, k, v, bias=bias, backend='hip')
+        held = torch.cuda.memory_allocated() - before
+        packed = B * 12 * 12 * 4096
+        assert held <= out.numel() * 2 + B * H * n * 4 + 4096 < packed
+        torch.autograd.grad(out, (q, bias) if want else q, torch.ones_like(out))
+
+
 def test_workspace_without_room_for_the_packed_bias():
     """A caller that passes no workspace to a mask-free forward with a shared
     bias is served by the general kernels, to rounding."""
