@@ -513,16 +513,16 @@ def _backward(prep: _Prepared, o, lse, fwd_ws, dout, want_dbias: bool, norm=None
     if norm is None:
         flags |= _lib.NXA_WS_PACK
     need = prep.workspace_bytes(flags)
-    ready = 0
+    ready, written = 0, 1 if norm is None else 2  # by nxa_fwd, nxa_fwd_normed
     if fwd_ws is not None and fwd_ws.numel() >= need:
         ws = fwd_ws
-        ready = 1 if prep.mask is not None else 0
+        ready = written if prep.mask is not None else 0
     else:
         ws = prep.workspace(flags)
         if prep.mask is not None and fwd_ws is not None:
             tm = prep.workspace_bytes(_lib.NXA_WS_FWD)
             ws[:tm].copy_(fwd_ws[:tm])
-            ready = 1
+            ready = written
     if norm is None:
         rc = lib.nxa_bwd(
             ctypes.byref(prep.desc), _ptr(q), _ptr(k), _ptr(v), _ptr(prep.bias),

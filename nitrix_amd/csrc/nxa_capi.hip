@@ -998,8 +998,11 @@ int run_bwd(const nxa_desc* d, const void* q, const void* k, const void* v,
       return NXA_OK;
     }
   }
-  // A forward on the short-sequence or key-split kernels leaves no tile map.
-  if (sg.ok || split_geom(d, bias != nullptr, mask != nullptr).ok) tilemap_ready = 0;
+  // A forward on the short-sequence or key-split kernels leaves no tile map
+  // (nxa_fwd_normed, which tilemap_ready 2 names, never runs on them).
+  if (!(na && tilemap_ready == 2) &&
+      (sg.ok || split_geom(d, bias != nullptr, mask != nullptr).ok))
+    tilemap_ready = 0;
   // 16-bit I/O: the dQ kernel computes -delta and -lse * log2(e) for its own
   // rows and runs first; the fp32 kernels have a pass of its own.
   const bool dq_first = d->io_dtype != NXA_F32;

@@ -320,3 +320,24 @@ def test_fused_qk_norm_random_configuration(seed):
         e = relerr(got.float().cpu().numpy(), want)
         print(f'  {nm} relerr {e:.2e}', flush=True)
         assert e <= tol, (nm, e)
+
+
+@pytest.mark.parametrize('s, t', [(128, 128), (20, 700)])
+def test_normed_backward_reuses_the_forward_tile_map(s, t):
+    """The fused qk-norm forward writes the mask's tile map at every length,
+    also where a plain forward would not: one map a training step."""
+    from nitrix_amd import _lib, scaled_dot_product_attention
+
+    g = torch.Generator(device=_dev()).manual_seed(1)
+    q = torch.randn(2, 4, s, 64, generator=g, device=_dev()).to(DT['bf16']).requires_grad_(True)
+    k = torch.randn(2, 4, t, 64, generator=g, device=_dev()).to(DT['bf16']).requires_grad_(True)
+    mask = (torch.arange(t, device=_dev()) < t - 40)[None, None, None]
+    _lib.profile_reset()
+    _lib.profile_enable(True)
+    out = scaled_dot_product_attention(q, k, k, mask=mask, qk_norm=True, backend='hip')
+    torch.autograd.grad(out, (q, k), torch.ones_like(out))
+    torch.cuda.synchronize()
+    _lib.profile_enable(False)
+    count = _lib.profile_read('tilemap')[1]
+    _lib.profile_reset()
+    assert count == 1
