@@ -372,14 +372,14 @@ class _ScanHip(torch.autograd.Function):
     are already contiguous in the scan's dtype) and the saved sub-chunk states are
     kept with ``save_for_backward``, so an in-place change of an input
     between forward and backward raises torch's version-counter error; the
-    backward is not itself differentiable."""
+    backward is not itself differentiable.  ``train`` says whether a backward
+    can follow."""
 
     @staticmethod
-    def forward(ctx, x, delta, A, B, C, D):
-        keep = any(ctx.needs_input_grad)
-        prep = _ScanPrep(x, delta, A, B, C, D, keep)
-        y, state = _scan_forward(prep, keep)
-        if keep:
+    def forward(ctx, x, delta, A, B, C, D, train):
+        prep = _ScanPrep(x, delta, A, B, C, D, train)
+        y, state = _scan_forward(prep, train)
+        if train:
             ctx.save_for_backward(prep.x, prep.delta, prep.A, prep.B, prep.C, prep.D, state)
             for name in ('x', 'delta', 'A', 'B', 'C', 'D'):
                 setattr(prep, name, None)
@@ -405,6 +405,7 @@ class _ScanHip(torch.autograd.Function):
                 g = _unbroadcast(g.reshape(*lead, prep.length, prep.n), shape)
             out.append(g.to(dtype))
         out.append(None if dD is None or not ctx.needs_input_grad[5] else dD.to(prep.D_dtype))
+        out.append(None)
         return tuple(out)
 
 
@@ -421,7 +422,12 @@ def selective_scan_hip(
     supported set; differentiable in every input."""
     _check_tileable(x, delta, A, B, C, D)
     _lib.lib()  # a missing library is an error here, not a fallback
-    return _ScanHip.apply(x, delta, A, B, C, D)
+    # (inside the Function gradients are off, and needs_input_grad is set
+    # also under no_grad: whether a backward can follow is seen here)
+    train = torch.is_grad_enabled() and any(
+        t is not None and t.requires_grad for t in (x, delta, A, B, C, D)
+    )
+    return _ScanHip.apply(x, delta, A, B, C, D, train)
 
 
 def selective_scan(

@@ -13,7 +13,7 @@ import pytest
 import torch
 from _golden import load_golden
 
-from nitrix_amd import _lib
+from nitrix_amd import _lib, ssm
 from nitrix_amd._backend import NitrixBackendError, NitrixBackendFallback, reset_fallback_state
 from nitrix_amd.attention import HipNotTileable
 from nitrix_amd.ssm import (
@@ -118,6 +118,31 @@ def test_entry_points_reject_small_or_misaligned_workspace(lib):
     assert lib.nxa_ssm_fwd(1, 64, 8, 4, *f, base, None, base, need - 1, None) == _lib.NXA_E_WORKSPACE
     assert lib.nxa_ssm_fwd(1, 64, 8, 4, *f, base, None, base + 4, need, None) == _lib.NXA_E_WORKSPACE
     assert lib.nxa_ssm_fwd(1, 64, 8, 4, base + 2, *f[1:], base, None, base, need, None) == _lib.NXA_E_LAYOUT
+
+
+@pytest.mark.parametrize('grad, leaf, train', [
+    (True, True, True), (True, False, False), (False, True, False), (False, False, False),
+])
+def test_a_call_is_training_only_where_a_backward_can_follow(monkeypatch, grad, leaf, train):
+    # Inference of a module under no_grad: its parameters require gradients,
+    # the call keeps no states and takes the engine of an inference call.
+    seen = []
+
+    def forward(prep, keep_state):
+        seen.append((prep.fused, keep_state))
+        return torch.zeros(prep.nb, prep.length, prep.d), torch.zeros(1) if keep_state else None
+
+    monkeypatch.setattr(ssm, '_scan_forward', forward)
+    monkeypatch.setattr(ssm, '_check_tileable', lambda *a: None)
+    monkeypatch.setattr(ssm._lib, 'lib', lambda: None)
+    x, delta = torch.rand(1, 3000, 8), torch.rand(1, 3000, 8)
+    B, C = torch.rand(1, 3000, 16), torch.rand(1, 3000, 16)
+    A = -torch.rand(8, 16).requires_grad_(leaf)
+    with torch.set_grad_enabled(grad):
+        y = ssm.selective_scan_hip(x, delta, A, B, C)
+    assert y.requires_grad == train
+    # (a training step this long and narrow keeps the chunk-parallel kernels)
+    assert seen == [(not train, train)]
 
 
 # --- reference engine ---------------------------------------------------------
