@@ -652,9 +652,9 @@ int check_scan(int64_t nb, int32_t L, int32_t Dm, int32_t N, int32_t dtype) {
     return fail(NXA_E_UNSUPPORTED, "fused selective scan: state dim n=%d exceeds %d", N,
                 nxa::kScanMaxStates);
   // A chunk's rows, and the states of one step, are addressed with 32-bit
-  // byte offsets below 2^31; the backward's grid is one block per channel
-  // group of at least 8 channels.
-  if (Dm >= 1 << 24 || nb * (((int64_t)Dm + 3) / 4) >= (int64_t)1 << 30)
+  // byte offsets below 2^31; a grid holds less than 2^32 threads (blocks of
+  // 256 with four states a lane, the largest grids).
+  if (Dm >= 1 << 24 || nb * nxa::scan_groups(Dm, nxa::scan_padded_states(N), 4) > ((int64_t)1 << 24) - 8)
     return fail(NXA_E_SHAPE, "fused selective scan: nb=%lld d=%d exceed the grid", (long long)nb,
                 Dm);
   return NXA_OK;

@@ -238,17 +238,34 @@ def _unbroadcast(g: torch.Tensor, shape) -> torch.Tensor:
 def _takes_fused(nb: int, length: int, d: int, n: int, train: bool) -> bool:
     """Whether ``nxa_ssm_io_*`` take the call, else ``nxa_ssm_*``.
 
-    They hold up to 16 states and 32-bit offsets.  One block walks the whole
-    sequence of its channels, so a training step on a long sequence of few
-    channels (which leaves most CUs idle) takes 47.5 ns a step (batch 1, d
-    512, n 16, L 8192: 399 us), where the chunk-parallel kernels take about
-    70 us + 18 ns a step + 1.3 us per million state steps (290 us): they keep
-    L > 2400 + 4e-5 (state steps).  At L 2048 the fused kernels lead (109 us
-    against 133), with more channels too (batch 4: 598 against 725)."""
-    if n > _MAX_IO_STATES or d >= 1 << 24 or nb * (d // 4 + 1) >= 1 << 30:
-        return False
+    They hold up to 16 states, 32-bit offsets and a grid of below 2^32 threads.
+    One block walks the whole sequence of its channels, so a training step on
+    a long sequence of few channels (which leaves most CUs idle) takes 47.5 ns
+    a step (batch 1, d 512, n 16, L 8192: 399 us), where the chunk-parallel
+    kernels take about 70 us + 18 ns a step + 1.3 us per million state steps
+    (290 us): they keep L > 2400 + 4e-5 (state steps).  At L 2048 the fused
+    kernels lead (109 us against 133), with more channels too (batch 4: 598
+    against 725).
+
+    They pad the states to 8 or 16, the others to 4 too: up to 4 states cost
+    them twice the work and memory.  So up to 3 states train on the others
+    (what a step keeps stays below one state trajectory), and with up to 4 the
+    fused kernels keep the calls that their fewer launches decide, or that
+    give every CU two blocks of four states a lane (n 4, us, others -> fused:
+    training batch 8, d 1024, L 1024: 134 -> 126, L 2048: 253 -> 281; d 2048,
+    L 4096: 883 -> 848; inference d 1024, L 2048: 87 -> 79, L 4096: 182 ->
+    204; batch 1, d 16, L 4096: 45.8 -> 45.1, L 8192: 73 -> 85)."""
     states = 8 if n <= 8 else 16
-    return not train or length <= 2400 + 4e-5 * nb * length * d * states
+    groups = nb * -(-d // (256 // states))  # blocks of four states a lane
+    if n > _MAX_IO_STATES or d >= 1 << 24 or groups > (1 << 24) - 8:
+        return False
+    if n <= 4 and groups < 512:
+        size = nb * length * d
+        if train and (n < 4 or size > 15e6):
+            return False
+        if not train and (size > 25e6 or (length > 4096 and nb * d < 512)):
+            return False
+    return not train or (n >= 4 and length <= 2400 + 4e-5 * nb * length * d * states)
 
 
 class _ScanPrep:

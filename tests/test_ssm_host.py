@@ -145,6 +145,78 @@ def test_a_call_is_training_only_where_a_backward_can_follow(monkeypatch, grad, 
     assert seen == [(not train, train)]
 
 
+def test_engine_choice():
+    f = ssm._takes_fused
+    # more states than 16, and grids of 2^32 threads and more
+    assert not f(1, 64, 8, 17, False)
+    assert f(1 << 19, 1, 256, 16, False) and not f(1 << 20, 1, 256, 16, False)
+    # training on a long sequence of few channels
+    assert f(1, 2400, 512, 16, True) and not f(1, 8192, 512, 16, True)
+    assert f(1, 8192, 512, 16, False)
+    # one to four states: three train on the chunk-parallel kernels, four
+    # where the walk of padded states costs more than its launches save
+    assert not f(8, 256, 64, 3, True) and f(8, 256, 64, 3, False)
+    assert f(8, 1024, 1024, 4, True) and not f(8, 2048, 1024, 4, True)
+    assert f(8, 4096, 2048, 4, True) and f(8, 4096, 2048, 4, False)
+    assert f(8, 2048, 1024, 4, False) and not f(8, 4096, 1024, 4, False)
+    assert f(1, 4096, 16, 1, False) and not f(1, 8192, 16, 1, False)
+
+
+def _a256(x):
+    return (x + 255) // 256 * 256
+
+
+@pytest.mark.parametrize('nb, length, d, n', [
+    (1, 1, 1, 1), (2, 100, 300, 5), (8, 2048, 1536, 16), (4, 1023, 1200, 8), (16, 40, 2048, 8),
+])
+def test_fused_state_and_workspace_sizes(lib, nb, length, d, n):
+    np_, ns = (8 if n <= 8 else 16), -(-length // 8)
+    assert lib.nxa_ssm_io_state_bytes(nb, length, d, n) == nb * ns * np_ * d * 4
+    # four states a lane where that gives 512 blocks of one wave's channels, else two
+    npl = 4 if nb * -(-d // (64 * 4 // np_)) >= 512 else 2
+    groups = -(-d // (64 * npl // np_))
+    part = _a256(groups * nb * length * 2 * np_ * 4)
+    assert lib.nxa_ssm_io_workspace_bytes(nb, length, d, n) == (
+        part + _a256(nb * np_ * d * 4) + _a256(nb * d * 4))
+
+
+@pytest.mark.parametrize('nb, length, d, n', [
+    (2, 128, 8, 4), (2, 128, 8, 3), (4, 2048, 512, 1), (4, 2048, 512, 2), (4, 2048, 512, 4),
+    (4, 2048, 512, 8), (1, 8192, 2048, 16), (8, 2048, 1536, 16),
+])
+def test_no_state_trajectory_in_memory_on_the_chosen_engine(lib, nb, length, d, n):
+    # As test_no_state_trajectory_in_memory, over the entry points that a
+    # training step of this shape calls.
+    dims = (nb, length, d, n)
+    if ssm._takes_fused(*dims, True):
+        held = lib.nxa_ssm_io_state_bytes(*dims) + lib.nxa_ssm_io_workspace_bytes(*dims)
+    else:
+        held = lib.nxa_ssm_state_bytes(*dims) + max(
+            lib.nxa_ssm_workspace_bytes(*dims, b) for b in (0, 1))
+    assert held < nb * length * d * n * 4
+
+
+def test_fused_entry_points_check_their_arguments(lib):
+    F, dims = _lib.NXA_F32, (1, 64, 8, 4)
+    assert lib.nxa_ssm_io_fwd(*dims, F, *([None] * 9)) == _lib.NXA_E_ARG
+    assert lib.nxa_ssm_io_bwd(*dims, F, *([None] * 15), 0, None) == _lib.NXA_E_ARG
+    assert lib.nxa_ssm_io_fwd(1, 64, 8, 17, F, *([None] * 9)) == _lib.NXA_E_UNSUPPORTED
+    assert lib.nxa_ssm_io_fwd(*dims, 7, *([None] * 9)) == _lib.NXA_E_DTYPE
+    assert lib.nxa_ssm_io_fwd(0, 64, 8, 4, F, *([None] * 9)) == _lib.NXA_E_SHAPE
+    assert lib.nxa_ssm_io_fwd(1 << 20, 1, 256, 16, F, *([None] * 9)) == _lib.NXA_E_SHAPE
+    assert lib.nxa_ssm_io_state_bytes(1, 64, 8, 17) == 0
+    assert lib.nxa_ssm_io_workspace_bytes(1, 64, 8, 17) == 0
+    host = np.zeros(1 << 16, np.uint8)
+    base = (host.ctypes.data + 255) // 256 * 256  # (host addresses: never dereferenced)
+    need = lib.nxa_ssm_io_workspace_bytes(*dims)
+    p = [base] * 14  # x, delta, A, B, C, D, state, dy, dx, ddelta, dA, dB, dC, dD
+    assert lib.nxa_ssm_io_bwd(*dims, F, *p, base, need - 1, None) == _lib.NXA_E_WORKSPACE
+    assert lib.nxa_ssm_io_bwd(*dims, F, *p, base + 4, need, None) == _lib.NXA_E_WORKSPACE
+    assert lib.nxa_ssm_io_bwd(*dims, F, base + 2, *p[1:], base, need, None) == _lib.NXA_E_LAYOUT
+    q = [*p[:6], base + 8, *p[7:]]  # the states are 16-byte aligned
+    assert lib.nxa_ssm_io_bwd(*dims, F, *q, base, need, None) == _lib.NXA_E_LAYOUT
+
+
 # --- reference engine ---------------------------------------------------------
 
 
