@@ -155,6 +155,14 @@ __device__ __forceinline__ float sum_channels(const float (&v)[NPL]) {
   return s;
 }
 
+// A log2(e).  A rate of -inf becomes the lowest finite one: the same decays
+// (0 for every step above 1e-36), while the steps past the end of the
+// sequence, whose delta is 0, keep the decay 1 and not 0 * -inf.
+__device__ __forceinline__ float decay_rate(float a) {
+  const float r = a * kLog2e;
+  return r < -3.402823466e38f ? -3.402823466e38f : r;
+}
+
 // Block -> (batch, channel group): runs of neighbouring groups on one XCD,
 // whose L2 then serves the 128-byte lines that neighbours share.
 __device__ __forceinline__ bool scan_block(const ScanParams& p, int64_t& b, int& cg) {
@@ -256,7 +264,7 @@ __global__ __launch_bounds__(NW * 64, NPL == 4 ? 3 : 1) void scan_fwd_kernel(con
   float al[NPL], carry[NPL];
 #pragma unroll
   for (int i = 0; i < NPL; ++i) {
-    al[i] = n0 + i < p.N ? p.A[(int64_t)dc * p.N + n0 + i] * kLog2e : 0.f;
+    al[i] = n0 + i < p.N ? decay_rate(p.A[(int64_t)dc * p.N + n0 + i]) : 0.f;
     carry[i] = 0.f;
   }
   const float Dd = p.D ? p.D[dc] : 0.f;
@@ -377,7 +385,7 @@ __global__ __launch_bounds__(NW * 64, NPL == 4 && NP == 16 ? 3 : 2) void scan_bw
   float al[NPL], carry[NPL], dA[NPL];
 #pragma unroll
   for (int i = 0; i < NPL; ++i) {
-    al[i] = n0 + i < p.N ? p.A[(int64_t)dc * p.N + n0 + i] * kLog2e : 0.f;
+    al[i] = n0 + i < p.N ? decay_rate(p.A[(int64_t)dc * p.N + n0 + i]) : 0.f;
     carry[i] = dA[i] = 0.f;
   }
   const float Dd = p.D ? p.D[dc] : 0.f;

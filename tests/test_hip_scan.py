@@ -84,3 +84,28 @@ def test_seventeen_states_and_mixed_dtypes():
     y = selective_scan(*[t.to(dev) for t in (xb, delta, A, B, C)], backend='hip')
     ref = S.selective_scan(*[t.double().numpy() for t in (xb, delta, A, B, C)], None)
     assert np.linalg.norm(y.double().cpu().numpy() - ref) / np.linalg.norm(ref) <= 2e-6
+
+
+@pytest.mark.parametrize('length', [13, 16, 130])
+def test_an_infinite_decay_rate(length):
+    """States that forget at once (A = -inf, an overflowed exponential): the
+    other states' gradients do not see the padded steps of a ragged end."""
+    from nitrix_amd import selective_scan
+
+    dev, nb, d, n = torch.device('cuda:0'), 2, 20, 8
+    g = torch.Generator().manual_seed(length)
+    x, dy = torch.randn(nb, length, d, generator=g), torch.randn(nb, length, d, generator=g)
+    B, C = torch.randn(nb, length, n, generator=g), torch.randn(nb, length, n, generator=g)
+    delta = 0.01 + torch.rand(nb, length, d, generator=g)
+    A = -(0.2 + torch.rand(d, n, generator=g))
+    A[:, ::3] = -float('inf')
+    ins = [t.to(dev) for t in (x, delta, A, B, C)]
+    for i in (0, 3, 4):
+        ins[i].requires_grad_(True)
+    y = selective_scan(*ins, backend='hip')
+    got = [y, *torch.autograd.grad(y, [ins[i] for i in (0, 3, 4)], dy.to(dev))]
+    a64 = [t.double().numpy() for t in (x, delta, A.clamp(min=-1e30), B, C)]
+    vjp = S.selective_scan_vjp(*a64, None, dy.double().numpy())
+    for a, w in zip(got, [S.selective_scan(*a64, None), vjp[0], vjp[3], vjp[4]]):
+        a = a.detach().double().cpu().numpy()
+        assert np.linalg.norm(a - w) <= TOL['f32'] * np.linalg.norm(w)
