@@ -692,8 +692,11 @@ __global__ __launch_bounds__(256, SPLIT ? 2 : 1) void dkdv32_kernel(const Params
     const int q0 = t * BQ;
     if constexpr (SPLIT) {
       // Only this wave reads its stage: its own wait publishes the copies.
+      // (The wait is no memory operation to the compiler and no barrier
+      // follows: the fences keep the LDS reads on its right side.)
       issue(i, st);
       __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+      asm volatile("" ::: "memory");
     } else {
       issue(i + 1, st ^ 1);
     }
@@ -873,6 +876,7 @@ __global__ __launch_bounds__(256, SPLIT ? 2 : 1) void dkdv32_kernel(const Params
 
     if constexpr (SPLIT) {
       // The next copies overwrite the stage the products just read.
+      asm volatile("" ::: "memory");
       __builtin_amdgcn_s_waitcnt(lgkmcnt_imm(0));
     } else {
       // Tile i + 1 is resident, and every wave is done with stage st, before
@@ -1033,8 +1037,11 @@ __global__ __launch_bounds__(256, SPLIT ? 2 : 1) void dq32_kernel(const Params p
     const int k0 = t * BN;
     if constexpr (SPLIT) {
       // Only this wave reads its stage: its own wait publishes the copies.
+      // (The wait is no memory operation to the compiler and no barrier
+      // follows: the fences keep the LDS reads on its right side.)
       issue(i, st);
       __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+      asm volatile("" ::: "memory");
     } else {
       issue(i + 1, st ^ 1);
     }
@@ -1134,6 +1141,7 @@ __global__ __launch_bounds__(256, SPLIT ? 2 : 1) void dq32_kernel(const Params p
 
     if constexpr (SPLIT) {
       // The next copies overwrite the stage the products just read.
+      asm volatile("" ::: "memory");
       __builtin_amdgcn_s_waitcnt(lgkmcnt_imm(0));
     } else {
       __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
