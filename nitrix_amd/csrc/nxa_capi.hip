@@ -309,6 +309,9 @@ ShortGeom short_geom(const nxa_desc* d, int has_bias, int has_mask) {
     g.OH = d->bias_str[1] == 0 ? 1 : d->H;
     const int64_t slots = (int64_t)g.OB * g.OH;
     if ((int64_t)d->B * d->H < 4 * slots) g.ok = false;
+    // The sum of dbias runs a thread per element of every slot, and a grid
+    // holds less than 2^32 threads.
+    if (slots * g.nqb * g.nkb * 1024 >= (int64_t)1 << 32) g.ok = false;
     g.pack_bytes = (size_t)slots * g.nqb * g.nkb * 1024 * sizeof(float);
     g.fwd_pack = g.ok && fwd_pays_pack(d, slots);
     g.bwd_pack = g.ok && bwd_pays_pack(d);

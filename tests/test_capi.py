@@ -356,3 +356,13 @@ def test_room_for_a_packed_bias_only_where_packing_pays(lib, B, H, shared, L, D,
     base = lib.nxa_workspace_bytes(ctypes.byref(d), 1, 0, _lib.NXA_WS_FWD)
     room = lib.nxa_workspace_bytes(ctypes.byref(d), 1, 0, _lib.NXA_WS_PACK) - base
     assert room == (slots * tiles * 4096 if packs else 0)
+
+
+@pytest.mark.parametrize('B, packs', [(16383, True), (16384, False)])
+def test_biases_of_a_full_grid_stay_with_the_general_kernels(lib, B, packs):
+    # One thread per element of 16384 biases of 512 x 512 is a grid of 2^32.
+    d = _desc(B, 4, 512, 512, 32)
+    d.bias_str[:] = (512 * 512, 0, 512)
+    flags = _lib.NXA_WS_BWD | _lib.NXA_WS_DBIAS
+    base = lib.nxa_workspace_bytes(ctypes.byref(d), 1, 0, flags)
+    assert (lib.nxa_workspace_bytes(ctypes.byref(d), 1, 0, flags | _lib.NXA_WS_PACK) > base) == packs
