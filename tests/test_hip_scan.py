@@ -66,6 +66,48 @@ def test_chunks_groups_and_states(name, nb, length, d, n):
     _check(name, nb, length, d, n, with_d=n % 2 == 0, seed=length)
 
 
+@pytest.mark.parametrize('name', ['f32', 'bf16', 'f16'])
+@pytest.mark.parametrize('nb, length, d, n, eight', [
+    (30, 20, 145, 8, True), (30, 300, 137, 5, True), (40, 33, 60, 16, True), (40, 129, 58, 9, True),
+    (25, 20, 145, 8, False), (32, 20, 60, 16, False),
+])
+def test_both_sides_of_the_eight_wave_rule(name, nb, length, d, n, eight):
+    """Blocks of 8 waves (one state a lane forward, two backward) where more
+    than 512 forward and 256 backward blocks fill the chip without 16; below,
+    blocks of 16."""
+    np_ = 8 if n <= 8 else 16
+
+    def groups(states):  # blocks with so many states a lane
+        return nb * -(-d // (64 * states // np_))
+
+    assert groups(4) < 512
+    assert (groups(1) > 512) == (groups(2) > 256) == eight
+    _check(name, nb, length, d, n, seed=length + d)
+
+
+@pytest.mark.parametrize('name', ['f32', 'bf16', 'f16'])
+@pytest.mark.parametrize('nb, length, d, n', [
+    (1, 1, 1, 1), (2, 7, 5, 3), (1, 33, 17, 2), (3, 100, 300, 4), (1, 129, 33, 5), (2, 33, 257, 16),
+    (2, 96, 128, 8), (1, 257, 64, 12), (700, 20, 9, 16), (1, 700, 40, 8),
+])
+@pytest.mark.parametrize('fused', [False, True], ids=['chunked', 'fused'])
+def test_either_engine(monkeypatch, name, nb, length, d, n, fused):
+    """Both engines at up to 16 states, whichever the host rule would take."""
+    from nitrix_amd import ssm
+
+    monkeypatch.setattr(ssm, '_takes_fused', lambda *a: fused)
+    _check(name, nb, length, d, n, with_d=n % 2 == 0, seed=length)
+
+
+@pytest.mark.parametrize('n', [8, 16])
+@pytest.mark.parametrize('length, fused', [(2400, True), (2500, False)])
+def test_the_engine_of_a_long_training_step(length, fused, n):
+    from nitrix_amd import ssm
+
+    assert ssm._takes_fused(1, length, 12, n, True) == fused
+    _check('f32', 1, length, 12, n, seed=n)
+
+
 @pytest.mark.parametrize('name, length', [('f32', 2400), ('bf16', 2403), ('f32', 2600)])
 def test_both_sides_of_the_long_sequence_rule(name, length):
     _check(name, 1, length, 12, 4, seed=length)

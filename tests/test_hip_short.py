@@ -116,6 +116,55 @@ def test_large_finite_bias_as_a_mask(dtype, bias_dtype, d, const):
         assert err <= tol, (name, err)
 
 
+@pytest.mark.parametrize('dtype, d, dv', [(BF, 64, 64), (HF, 40, 56)], ids=['bf16', 'f16'])
+@pytest.mark.parametrize('s, t', [(343, 343), (511, 449)])
+@pytest.mark.parametrize('kind', ['plain', 'causal', 'keypad', 'bias'])
+def test_eight_wave_blocks(dtype, d, dv, s, t, kind):
+    """Blocks of 8 waves in the forward, dQ and dK / dV: more than 53 KB
+    resident and more than 256 blocks of 128 rows (the launcher's rule; a
+    bias of odd rows is packed in the forward too)."""
+    B, H = 24, 4
+    for resident, strips in ((t, s), (s, t)):
+        assert 2 * -(-resident // 64) * 64 * 64 * 2 > 53 * 1024
+        assert B * H * -(-strips // 128) > 256
+    kw = {'plain': {}, 'causal': dict(causal=True), 'keypad': dict(mask_kind='keypad'),
+          'bias': dict(bias_shape=(1, H, s, t), bias_dtype=F32)}[kind]
+    _check(dtype, B, H, s, t, d, dv=dv, seed=s + d, **kw)
+
+
+@pytest.mark.parametrize('L, d', [(296, 32), (304, 64)])
+def test_packed_forward_of_aligned_bias_rows(L, d):
+    """A bias the general forward could read as it is, packed where enough
+    pairs share it."""
+    B, H = 33, 8
+    from nitrix_amd import _lib
+    from nitrix_amd.attention import _Prepared
+
+    q = torch.zeros(B, H, L, d, device=_dev(), dtype=BF)
+    bias = torch.zeros(1, H, L, L, device=_dev(), dtype=BF)
+    prep = _Prepared(q, q, q, bias, None, d ** -0.5, False)
+    assert prep.workspace_bytes(_lib.NXA_WS_PACK) > prep.workspace_bytes(_lib.NXA_WS_FWD)
+    _check(BF, B, H, L, L, d, bias_shape=(1, H, L, L), seed=L, grads=False)
+    _check(BF, B, H, L, L, d, bias_shape=(1, H, L, L), causal=True, mask_kind='keypad', seed=L,
+           grads=False)
+
+
+def test_a_call_repeats_itself():
+    from nitrix_amd import scaled_dot_product_attention
+
+    g = torch.Generator(device=_dev()).manual_seed(2)
+    q, k, v, do = (torch.randn(16, 4, 343, 32, generator=g, device=_dev()).to(BF) for _ in range(4))
+    bias = torch.randn(1, 4, 343, 343, generator=g, device=_dev()).to(BF)
+    ins = [t.requires_grad_(True) for t in (q, k, v, bias)]
+    runs = []
+    for _ in range(3):
+        out = scaled_dot_product_attention(q, k, v, bias=bias, backend='hip')
+        runs.append((out, *torch.autograd.grad(out, ins, do)))
+    for run in runs[1:]:
+        for a, b in zip(runs[0], run):
+            assert torch.equal(a, b)
+
+
 def test_the_packed_bias_is_not_kept_for_the_backward():
     """Between forward and backward a call holds its output, the row values
     and no packed bias (which is larger than the bias itself)."""

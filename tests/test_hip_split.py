@@ -81,3 +81,13 @@ def test_scores_of_minus_infinity(dtype, t):
     ref = O.sdpa_forward(q[:, :, rows], k, v, mask=mask, scale=d ** -0.5, acc_dtype=np.float64)
     assert np.isfinite(got).all()
     assert np.abs(got - ref).max() / np.abs(ref).max() <= (2e-2 if dtype == BF else 2e-3)
+
+
+def test_a_call_repeats_itself():
+    from nitrix_amd import scaled_dot_product_attention
+
+    g = torch.Generator(device=_dev()).manual_seed(2)
+    q, k, v = (torch.randn(4, 8, n, 64, generator=g, device=_dev()).to(HF) for n in (28, 8192, 8192))
+    mask = (torch.arange(8192, device=_dev()) < 7001)[None, None, None]
+    outs = [scaled_dot_product_attention(q, k, v, mask=mask, backend='hip') for _ in range(3)]
+    assert all(torch.equal(outs[0], o) for o in outs[1:])
