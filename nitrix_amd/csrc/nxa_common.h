@@ -704,4 +704,50 @@ __device__ __forceinline__ int xcd_remap(int bid, int nheads, int ntiles) {
   return (x + kXcd * (k / ntiles)) * ntiles + k % ntiles;
 }
 
+__device__ __forceinline__ f32x16 splat16(float x) {
+  f32x16 r;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) r[i] = x;
+  return r;
+}
+
+// Row and transposed fragment reads of swizzled [rows x DP] LDS tiles (see
+// nxa_fwd16.h).
+template <typename T, int DP>
+struct Resident {
+  using Frag = typename Mma<T>::Frag;
+  static constexpr int NC = DP / 16, NDB = DP / 32;
+  uint32_t row_off[NC];
+  uint32_t tr_off[NDB][2];
+  __device__ __forceinline__ void init(int lane) {
+    const int g = lane >> 5, c32 = lane & 31;
+#pragma unroll
+    for (int m = 0; m < NC; ++m) row_off[m] = 2 * swz_off<DP>(c32, 2 * m + g);
+    const int tr_row = 4 * ((lane >> 4) >> 1) + ((lane & 15) >> 2);
+    const int tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+        const int col = db * 32 + tr_col;
+        tr_off[db][hh] = 2 * (swz_off<DP>(tr_row + 8 * hh, col >> 3) + (col & 7));
+      }
+  }
+  // Head-dim chunk m of the 32 rows from byte offset `at` (a multiple of 32 rows).
+  __device__ __forceinline__ Frag row(uint32_t at, int m) const {
+    typedef __attribute__((address_space(3))) Frag lds_frag;
+    return *(const lds_frag*)(uintptr_t)(at + row_off[m]);
+  }
+  // Transposed fragment f (16 rows) of those rows, head-dim block db.
+  __device__ __forceinline__ Frag tr(uint32_t at, int f, int db) const {
+    typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+    typedef short i16x8 __attribute__((ext_vector_type(8)));
+    const uint32_t ro = at + f * (16 * DP * 2);
+    const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(uintptr_t)(ro + tr_off[db][0]));
+    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(uintptr_t)(ro + tr_off[db][1]));
+    const i16x8 r = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    return __builtin_bit_cast(Frag, r);
+  }
+};
+
 }  // namespace nxa

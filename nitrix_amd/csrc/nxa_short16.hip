@@ -88,44 +88,6 @@ __device__ __forceinline__ void load_resident(const T* src, int64_t rs, int nrow
   }
 }
 
-// Row and transposed fragment reads of a resident matrix (see nxa_fwd16.h).
-template <typename T, int DP>
-struct Resident {
-  using Frag = typename Mma<T>::Frag;
-  static constexpr int NC = DP / 16, NDB = DP / 32;
-  uint32_t row_off[NC];
-  uint32_t tr_off[NDB][2];
-  __device__ __forceinline__ void init(int lane) {
-    const int g = lane >> 5, c32 = lane & 31;
-#pragma unroll
-    for (int m = 0; m < NC; ++m) row_off[m] = 2 * swz_off<DP>(c32, 2 * m + g);
-    const int tr_row = 4 * ((lane >> 4) >> 1) + ((lane & 15) >> 2);
-    const int tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-#pragma unroll
-    for (int db = 0; db < NDB; ++db)
-#pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        const int col = db * 32 + tr_col;
-        tr_off[db][hh] = 2 * (swz_off<DP>(tr_row + 8 * hh, col >> 3) + (col & 7));
-      }
-  }
-  // Head-dim chunk m of the 32 rows from byte offset `at` (a multiple of 32 rows).
-  __device__ __forceinline__ Frag row(uint32_t at, int m) const {
-    typedef __attribute__((address_space(3))) Frag lds_frag;
-    return *(const lds_frag*)(uintptr_t)(at + row_off[m]);
-  }
-  // Transposed fragment f (16 rows) of those rows, head-dim block db.
-  __device__ __forceinline__ Frag tr(uint32_t at, int f, int db) const {
-    typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
-    typedef short i16x8 __attribute__((ext_vector_type(8)));
-    const uint32_t ro = at + f * (16 * DP * 2);
-    const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(uintptr_t)(ro + tr_off[db][0]));
-    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(uintptr_t)(ro + tr_off[db][1]));
-    const i16x8 r = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    return __builtin_bit_cast(Frag, r);
-  }
-};
-
 // Row fragments of one 32-row strip of a [n, D] matrix in memory.
 template <int NC, typename T>
 __device__ __forceinline__ void strip_frags(typename Mma<T>::Frag (&f)[NC], const T* row, bool ok,
@@ -135,13 +97,6 @@ __device__ __forceinline__ void strip_frags(typename Mma<T>::Frag (&f)[NC], cons
     const int d = c * 16 + g * 8;
     f[c] = ok && d < D ? ld16(row + d) : zero_frag<T>();
   }
-}
-
-__device__ __forceinline__ f32x16 splat16(float x) {
-  f32x16 r;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) r[i] = x;
-  return r;
 }
 
 // Packed bias block (32 x 32) as a score accumulator.
@@ -517,7 +472,8 @@ __global__ __launch_bounds__(NW * 64, 2) void dq_short_kernel(const Params p, co
 // 32-key strips.  Rows past Lq read as zeros with -lse2 = -inf, so P = 0.
 // ---------------------------------------------------------------------------
 template <typename T, int DP, int NW, bool HAS_BIAS, bool CAUSAL>
-__global__ __launch_bounds__(NW * 64, DP == 32 && !CAUSAL ? 4 : 2) void dkdv_short_kernel(const Params p, const ShortParams sp) {
+__global__ __launch_bounds__(NW * 64, DP == 32 && !CAUSAL ? 4 : 2) void dkdv_short_kernel(
+    const Params p, const ShortParams sp) {
   using M = Mma<T>;
   using Frag = typename M::Frag;
   constexpr int NC = DP / 16, NDB = DP / 32, FPB = M::FRAGS_PER_BLOCK;
@@ -654,7 +610,6 @@ constexpr int kDbiasWaves = DP == 32 ? 4 : 8;
 template <typename T, int DP, bool CAUSAL>
 __global__ __launch_bounds__(kDbiasWaves<DP> * 64, DP == 32 ? 3 : 2) void dbias_pairs_kernel(const Params p, const ShortParams sp) {
   using M = Mma<T>;
-  using Frag = typename M::Frag;
   constexpr int NC = DP / 16, SPR = DP / 8, NST = 2;
   constexpr int NW = kDbiasWaves<DP>, BK = NW * 16;
   constexpr int MAT = 128 * DP * 2, KMAT = BK * DP * 2, HALF = 32 * DP * 2;

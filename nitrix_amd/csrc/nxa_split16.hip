@@ -27,13 +27,6 @@ namespace {
 constexpr int kSplitWaves = 4;
 constexpr int kSplitTiles = 64;  // most tiles a wave lists
 
-__device__ __forceinline__ f32x16 zero16() {
-  f32x16 r;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) r[i] = 0.f;
-  return r;
-}
-
 // Weights of N partial results with reference maxima m (all -inf: zeros).
 template <int N>
 __device__ __forceinline__ float merge_weights(const float (&m)[N], float (&sc)[N]) {
@@ -167,26 +160,12 @@ __global__ __launch_bounds__(256, 2) void fwd_split_kernel(const Params p, const
     }
   };
 
-  // LDS read offsets (see nxa_fwd16.h).
-  uint32_t row_off[NC], tr_off[NDB][2];
-#pragma unroll
-  for (int m = 0; m < NC; ++m) row_off[m] = 2 * swz_off<DP>(c32, 2 * m + g);
-  const int tr_row = 4 * ((lane >> 4) >> 1) + ((lane & 15) >> 2);
-  const int tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-#pragma unroll
-  for (int db = 0; db < NDB; ++db)
-#pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-      const int col = db * 32 + tr_col;
-      tr_off[db][hh] = 2 * (swz_off<DP>(tr_row + 8 * hh, col >> 3) + (col & 7));
-    }
-  typedef __attribute__((address_space(3))) Frag lds_frag;
-  typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
-  typedef short i16x8 __attribute__((ext_vector_type(8)));
+  Resident<T, DP> rd;
+  rd.init(lane);
 
   f32x16 oacc[NDB];
 #pragma unroll
-  for (int db = 0; db < NDB; ++db) oacc[db] = zero16();
+  for (int db = 0; db < NDB; ++db) oacc[db] = splat16(0.f);
   float m_ref = -INFINITY, l_i = 0.f;
   // The Q loads complete here, so the waits below only count tile copies.
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
@@ -201,7 +180,7 @@ __global__ __launch_bounds__(256, 2) void fwd_split_kernel(const Params p, const
     f32x16 s;
 #pragma unroll
     for (int m = 0; m < NC; ++m) {
-      const Frag a = *(const lds_frag*)(uintptr_t)(at + row_off[m]);
+      const Frag a = rd.row(at, m);
       if (m == 0) s = M::first(a, qf[m]);
       else M::run(s, a, qf[m]);
     }
@@ -239,13 +218,7 @@ __global__ __launch_bounds__(256, 2) void fwd_split_kernel(const Params p, const
     for (int f = 0; f < FPB; ++f) {
       const Frag pf = M::pack(s, f);
 #pragma unroll
-      for (int db = 0; db < NDB; ++db) {
-        const uint32_t ro = at + TILE + f * (16 * DP * 2);
-        const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(uintptr_t)(ro + tr_off[db][0]));
-        const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(uintptr_t)(ro + tr_off[db][1]));
-        const i16x8 r = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        M::run(oacc[db], __builtin_bit_cast(Frag, r), pf);
-      }
+      for (int db = 0; db < NDB; ++db) M::run(oacc[db], rd.tr(at + TILE, f, db), pf);
     }
     // The next copies overwrite the stage that these reads used.
     asm volatile("" ::: "memory");
