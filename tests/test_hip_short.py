@@ -149,6 +149,69 @@ def test_packed_forward_of_aligned_bias_rows(L, d):
            grads=False)
 
 
+def _forms(x, dtype):
+    """The same values under other strides: [B, L, H, D] memory, rows apart,
+    a slice of a longer sequence."""
+    B, H, L, D = x.shape
+    t = _to(x, dtype)
+    wide = torch.zeros(B, H, L, D + 16, device=_dev(), dtype=dtype)
+    wide[..., 8:8 + D] = t
+    long = torch.zeros(B, H, L + 5, D, device=_dev(), dtype=dtype)
+    long[:, :, 3:3 + L] = t
+    return {'plain': t, 'blhd': t.transpose(1, 2).contiguous().transpose(1, 2),
+            'rows': wide[..., 8:8 + D], 'slice': long[:, :, 3:3 + L]}
+
+
+@pytest.mark.parametrize('form', ['blhd', 'rows', 'slice'])
+@pytest.mark.parametrize('s, t, d, bias', [
+    (70, 131, 32, None), (70, 131, 64, 'heads'), (200, 131, 32, 'batch'), (28, 700, 64, None),
+])
+def test_strided_inputs(form, s, t, d, bias):
+    """Any strides give the bytes of contiguous inputs: outputs and gradients
+    of the short-sequence and key-split paths, a bias of spaced rows among them."""
+    from nitrix_amd import scaled_dot_product_attention
+
+    rng = np.random.default_rng(s + d)
+    B, H = 72, 4
+    fq, fk, fv, fg = (_forms(_draw(rng, (B, H, n, d), BF), BF) for n in (s, t, t, s))
+    b = None if bias is None else _draw(rng, {'heads': (1, H, s, t), 'batch': (B, 1, s, t)}[bias], BF)
+    runs = []
+    for f in ('plain', form):
+        ins = [x[f].detach().requires_grad_(True) for x in (fq, fk, fv)]
+        tb = None
+        if b is not None:
+            tb = _to(b, BF)
+            if f != 'plain':
+                tb = torch.nn.functional.pad(tb, (3, 2))[..., 3:3 + t].detach()
+            ins.append(tb.requires_grad_(True))
+        out = scaled_dot_product_attention(*ins[:3], bias=tb, backend='hip')
+        runs.append((out, *torch.autograd.grad(out, ins, fg[f])))
+    for a, c in zip(*runs):
+        assert torch.equal(a, c)
+
+
+@pytest.mark.parametrize('s, t', [(70, 131), (28, 700)])
+def test_inputs_broadcast_over_heads_and_batch(s, t):
+    """Keys shared by all heads, values by all batches, as views."""
+    from nitrix_amd import scaled_dot_product_attention
+
+    rng = np.random.default_rng(t)
+    B, H, d = 3, 4, 64
+    q, k, v, g = (_to(_draw(rng, sh, BF), BF, True) for sh in
+                  ((B, H, s, d), (B, 1, t, d), (1, H, t, d), (B, H, s, d)))
+    runs = []
+    for expand in (False, True):
+        ke, ve = k.expand(B, H, t, d), v.expand(B, H, t, d)
+        if not expand:
+            ke, ve = ke.contiguous(), ve.contiguous()
+        with torch.no_grad():
+            o = scaled_dot_product_attention(q, ke, ve, backend='hip')
+        out = scaled_dot_product_attention(q, ke, ve, backend='hip')
+        runs.append((o, out, *torch.autograd.grad(out, (q, k, v), g.detach())))
+    for a, c in zip(*runs):
+        assert torch.equal(a, c)
+
+
 def test_a_call_repeats_itself():
     from nitrix_amd import scaled_dot_product_attention
 
