@@ -235,8 +235,9 @@ def _unbroadcast(g: torch.Tensor, shape) -> torch.Tensor:
     return g
 
 
-def _takes_fused(nb: int, length: int, d: int, n: int, train: bool) -> bool:
-    """Whether ``nxa_ssm_io_*`` take the call, else ``nxa_ssm_*``.
+def _takes_fused(nb: int, length: int, d: int, n: int, train: bool, f32: bool = True) -> bool:
+    """Whether ``nxa_ssm_io_*`` take the call, else ``nxa_ssm_*`` (``f32``:
+    the former would read float32, as the latter always do).
 
     They hold up to 16 states, 32-bit offsets and a grid of below 2^32 threads.
     One block walks the whole sequence of its channels, so a training step on
@@ -245,7 +246,11 @@ def _takes_fused(nb: int, length: int, d: int, n: int, train: bool) -> bool:
     kernels take about 70 us + 18 ns a step + 1.3 us per million state steps
     (290 us): they keep L > 2400 + 4e-5 (state steps).  At L 2048 the fused
     kernels lead (109 us against 133), with more channels too (batch 4: 598
-    against 725).
+    against 725).  Past 6000 steps the chunk-parallel kernels also keep
+    float32 training of 9 to 16 states whose backward would leave a fifth of
+    the CUs idle in its rounds of one block a CU (L 8192, batch 1, d 1536, 192
+    blocks: 584 us against 526; d 2048, 256 blocks: 0.96 of their time; in 16
+    bits their upcasts cost more than that).
 
     They pad the states to 8 or 16, the others to 4 too: up to 4 states cost
     them twice the work and memory.  So up to 3 states train on the others
@@ -265,6 +270,11 @@ def _takes_fused(nb: int, length: int, d: int, n: int, train: bool) -> bool:
             return False
         if not train and (size > 25e6 or (length > 4096 and nb * d < 512)):
             return False
+    blocks = nb * -(-d // (128 // states))  # of two states a lane
+    idle = -blocks % 256
+    if (train and f32 and n > 8 and length > 6000 and groups < 512
+            and blocks > 128 and 5 * idle > blocks + idle):
+        return False
     return not train or (n >= 4 and length <= 2400 + 4e-5 * nb * length * d * states)
 
 
@@ -286,12 +296,15 @@ class _ScanPrep:
         bn = self.batch + (length, self.n)
         # The dtype the kernels read x, delta, B and C in (float32 also where
         # gradients of a broadcast B or C are summed over their copies).
-        self.fused = _takes_fused(self.nb, length, d, self.n, train)
         one = (
             x.dtype == delta.dtype == B.dtype == C.dtype
             and tuple(B.shape) == tuple(C.shape) == bn
+            and x.dtype in _HIP_DTYPES
         )
-        self.scan = x.dtype if self.fused and one and x.dtype in _HIP_DTYPES else f32
+        self.scan = x.dtype if one else f32
+        self.fused = _takes_fused(self.nb, length, d, self.n, train, self.scan == f32)
+        if not self.fused:
+            self.scan = f32
 
         def flat(t, shape, last):
             return t.to(self.scan).expand(shape).reshape(self.nb, length, last).contiguous()

@@ -153,6 +153,10 @@ def test_engine_choice():
     # training on a long sequence of few channels
     assert f(1, 2400, 512, 16, True) and not f(1, 8192, 512, 16, True)
     assert f(1, 8192, 512, 16, False)
+    # float32 training whose backward blocks leave CUs idle (192 of 256)
+    assert not f(1, 8192, 1536, 16, True) and f(1, 8192, 1536, 16, True, False)
+    assert f(1, 8192, 2048, 16, True) and f(1, 5000, 1536, 16, True)
+    assert f(2, 8192, 1536, 8, True)
     # one to four states: three train on the chunk-parallel kernels, four
     # where the walk of padded states costs more than its launches save
     assert not f(8, 256, 64, 3, True) and f(8, 256, 64, 3, False)
