@@ -447,13 +447,13 @@ def _forward(prep: _Prepared, for_bwd: bool = False, qnorm=None):
     lse = torch.empty(
         (prep.nb, prep.h, prep.s), dtype=torch.float32, device=prep.device
     )
-    ws, keep = None, True
+    need, keep = None, True
     if qnorm is None and _may_pack(prep):
-        room = prep.workspace_bytes(_lib.NXA_WS_PACK)
-        if room > prep.workspace_bytes(_lib.NXA_WS_FWD):
-            ws, keep = torch.empty(room, dtype=torch.uint8, device=prep.device), False
-    if keep:
-        ws = prep.workspace(_lib.NXA_WS_BWD if for_bwd else _lib.NXA_WS_FWD)
+        need = prep.workspace_bytes(_lib.NXA_WS_PACK)
+        keep = need == (0 if prep.mask is None else prep.workspace_bytes(_lib.NXA_WS_FWD))
+    if need is None or (keep and for_bwd):
+        need = prep.workspace_bytes(_lib.NXA_WS_BWD if for_bwd else _lib.NXA_WS_FWD)
+    ws = torch.empty(need, dtype=torch.uint8, device=prep.device) if need else None
     args = (ctypes.byref(prep.desc), _ptr(prep.q), _ptr(prep.k), _ptr(prep.v),
             _ptr(prep.bias), _ptr(prep.mask), _ptr(o), _ptr(lse))
     tail = (_ptr(ws), 0 if ws is None else ws.numel(), prep.stream())

@@ -270,12 +270,14 @@ def _takes_fused(nb: int, length: int, d: int, n: int, train: bool, f32: bool = 
             return False
         if not train and (size > 25e6 or (length > 4096 and nb * d < 512)):
             return False
-    blocks = nb * -(-d // (128 // states))  # of two states a lane
-    idle = -blocks % 256
-    if (train and f32 and n > 8 and length > 6000 and groups < 512
-            and blocks > 128 and 5 * idle > blocks + idle):
-        return False
-    return not train or (n >= 4 and length <= 2400 + 4e-5 * nb * length * d * states)
+    if not train:
+        return True
+    if f32 and n > 8 and length > 6000 and groups < 512:
+        blocks = nb * -(-d // (128 // states))  # of two states a lane
+        idle = -blocks % 256
+        if blocks > 128 and 5 * idle > blocks + idle:
+            return False
+    return n >= 4 and length <= 2400 + 4e-5 * nb * length * d * states
 
 
 class _ScanPrep:
