@@ -65,21 +65,21 @@ PEAK_HBM_GBS = 8000.0
 # TRAFFIC_SRC is the fingerprint (_src_fingerprint) of the attention kernel
 # sources the passes ran; when the sources differ, the figure describes other
 # kernels and is reported as stale (traffic null, the old figure beside it).
-TRAFFIC_SRC = '3424b6891ab6ff98'
+TRAFFIC_SRC = '6a3c003ef0b84fbd'
 MEASURED_TRAFFIC = {
-    'c1': ('fwd', 6102699),
-    'c2': ('dkdv', 910863461),
-    'c3': ('dkdv', 1619817728),
-    'c4': ('fwd', 4431318736),
-    'c5': ('dkdv', 706809013),
+    'c1': ('fwd', 6113962),
+    'c2': ('dkdv', 910714325),
+    'c3': ('dkdv', 1619918282),
+    'c4': ('fwd', 4431536352),
+    'c5': ('dkdv', 706633765),
 }
 # VALU instructions (wave64) of the selective scan's backward pass (both
 # kernels) per step at the ssm configuration, transcendental instructions
 # weighted 4: the rocprofv3 SQ_INSTS_VALU / SQ_INSTS_VALU_TRANS_F32 counts of its kernels in
 # profiles/selective_scan_valu_counters.md.
-SSM_BWD_VALU_WAVE_INSTS = 1.7965e8
+SSM_BWD_VALU_WAVE_INSTS = 1.7969e8
 # Fingerprint of nxa_scan.hip + nxa_common.h when the counts were taken.
-SSM_VALU_SRC = '7f743280a8be0215'
+SSM_VALU_SRC = '4bff318d224860e5'
 SSM_VALU_SOURCE = 'profiles/selective_scan_valu_counters.md (rocprofv3 SQ_INSTS_VALU, SQ_INSTS_VALU_TRANS_F32)'
 PEAK_VALU_TLANEOPS = 256 * 4 * 32 * 2.4e9 / 1e12  # 78.6 T lane-instructions/s
 TRAFFIC_SOURCE = 'profiles/attention_hbm_traffic_c1_c5.md (rocprofv3 FETCH_SIZE x2 + WRITE_SIZE x1)'

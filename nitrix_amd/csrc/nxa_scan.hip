@@ -35,7 +35,8 @@
 // here (forward 175 with its states, 150 without; backward 345; reduction
 // 35, bound by reading 200 MB of partial rows).  Batch 1, L 5000, d 1000,
 // n 16, bf16 forward: 121 -> 55 us (four upcasts, 44 us of serial carry).
-// The walk is bound by VALU issue; the saved states are written as whole
+// The walk is bound by VALU issue (VALU instructions are in issue 94 % of the
+// SIMDs' cycles in the backward, 76 % in the forward); the saved states are written as whole
 // lines (in [state][channel] order they cost 50 us more).
 #include "nxa_common.h"
 #include "nxa_launch.h"

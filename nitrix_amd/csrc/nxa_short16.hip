@@ -32,11 +32,13 @@
 // Measured (bf16, a bias [4, 343, 343] shared by 512 windows, head dim 32,
 // forward + backward): 4.62 ms on the general kernels (dK/dV 3.0 in twelve
 // launches with 284 us of reductions, the forward 0.78, dQ 0.55, both at
-// one bias element per load), 0.46 here: packs 2 x 5 us, forward 98, dQ 113,
-// dK/dV 126, dbias 149, its sum 6.  Without a bias (B 8, H 32, head dim 64,
+// one bias element per load), 0.42 here: packs 2 x 5 us, forward 104, dQ 115,
+// dK/dV 128, dbias 112, its sum 7.  Without a bias (B 8, H 32, head dim 64,
 // forward + backward on the GPU): 256 x 256 52 -> 42 us, 512 x 512 131 ->
-// 118; a lone 512 x 512 call of 16 heads 43 -> 42.  The kernels are bound by
-// VALU issue (one exponential and about five operations per score).
+// 118; a lone 512 x 512 call of 16 heads 43 -> 42.  The four kernels of the
+// windowed call are bound by VALU issue (one exponential and about five
+// operations per score): VALU instructions are in issue 54 to 60 % of the
+// SIMDs' cycles at two or three waves a SIMD, the matrix cores 16 to 27 %.
 #include "nxa_fwd16.h"
 #include "nxa_launch.h"
 
@@ -470,6 +472,8 @@ __global__ __launch_bounds__(NW * 64, 2) void dq_short_kernel(const Params p, co
 // ---------------------------------------------------------------------------
 // dK / dV: Q and dO resident (with their rows' -lse2 and -delta), waves take
 // 32-key strips.  Rows past Lq read as zeros with -lse2 = -inf, so P = 0.
+// (Four waves a SIMD at head dim 32: both loops' registers but for a few that
+// are written out once a strip.)
 // ---------------------------------------------------------------------------
 template <typename T, int DP, int NW, bool HAS_BIAS, bool CAUSAL>
 __global__ __launch_bounds__(NW * 64, DP == 32 && !CAUSAL ? 4 : 2) void dkdv_short_kernel(
