@@ -447,11 +447,14 @@ def _forward(prep: _Prepared, for_bwd: bool = False, qnorm=None):
     lse = torch.empty(
         (prep.nb, prep.h, prep.s), dtype=torch.float32, device=prep.device
     )
-    need, keep = None, True
+    keep = True
     if qnorm is None and _may_pack(prep):
         need = prep.workspace_bytes(_lib.NXA_WS_PACK)
-        keep = need == (0 if prep.mask is None else prep.workspace_bytes(_lib.NXA_WS_FWD))
-    if need is None or (keep and for_bwd):
+        if for_bwd:
+            keep = need == (0 if prep.mask is None else prep.workspace_bytes(_lib.NXA_WS_FWD))
+            if keep:
+                need = prep.workspace_bytes(_lib.NXA_WS_BWD)
+    else:
         need = prep.workspace_bytes(_lib.NXA_WS_BWD if for_bwd else _lib.NXA_WS_FWD)
     ws = torch.empty(need, dtype=torch.uint8, device=prep.device) if need else None
     args = (ctypes.byref(prep.desc), _ptr(prep.q), _ptr(prep.k), _ptr(prep.v),

@@ -456,8 +456,9 @@ def selective_scan_hip(
     _lib.lib()  # a missing library is an error here, not a fallback
     # (inside the Function gradients are off, and needs_input_grad is set
     # also under no_grad: whether a backward can follow is seen here)
-    train = torch.is_grad_enabled() and any(
-        t is not None and t.requires_grad for t in (x, delta, A, B, C, D)
+    train = torch.is_grad_enabled() and (
+        x.requires_grad or delta.requires_grad or A.requires_grad or B.requires_grad
+        or C.requires_grad or (D is not None and D.requires_grad)
     )
     return _ScanHip.apply(x, delta, A, B, C, D, train)
 
