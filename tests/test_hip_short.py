@@ -149,6 +149,30 @@ def test_packed_forward_of_aligned_bias_rows(L, d):
            grads=False)
 
 
+@pytest.mark.parametrize('dtype', [BF, HF], ids=['bf16', 'f16'])
+def test_a_large_positive_bias_takes_its_rows(dtype):
+    """One key at +1e9: every row's output is that key's value, its value's
+    gradient the sum of the cotangents, and no other gradient is larger than
+    the rounding of P (dP - delta)."""
+    from nitrix_amd import scaled_dot_product_attention
+
+    rng = np.random.default_rng(11)
+    B, H, s, t, d = 72, 4, 40, 131, 32
+    q, k, v, g = (_draw(rng, (B, H, n, d), dtype) for n in (s, t, t, s))
+    bias = _draw(rng, (1, H, s, t), F32)
+    bias[..., 77] = 1e9
+    tq, tk, tv = _to(q, dtype, True), _to(k, dtype, True), _to(v, dtype, True)
+    out = scaled_dot_product_attention(tq, tk, tv, bias=_to(bias, F32), backend='hip')
+    dq, dk, dv = (x.float().cpu().numpy() for x in
+                  torch.autograd.grad(out, (tq, tk, tv), _to(g, dtype)))
+    assert relerr(out.detach().float().cpu().numpy(), np.broadcast_to(v[:, :, 77:78], out.shape)) == 0
+    want = np.zeros_like(v, dtype=np.float64)
+    want[:, :, 77] = g.astype(np.float64).sum(2)
+    assert relerr(dv, want) <= REL[dtype]
+    # dP - delta: two sums of d products of unit size, in fp32
+    assert np.abs(dq).max() <= 1e-3 and np.abs(dk).max() <= s * 1e-3
+
+
 def _forms(x, dtype):
     """The same values under other strides: [B, L, H, D] memory, rows apart,
     a slice of a longer sequence."""
